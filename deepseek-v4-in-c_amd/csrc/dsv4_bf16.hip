@@ -164,6 +164,20 @@ void b16_launch(const B16Geom &g, float *y, const float *x, const uint16_t *W, i
                        rows, cols, g.tc, p.rows_per_wg, ls);
 }
 
+/* From how many tokens the batch runs on the f32 matrix core
+ * (dsv4_batch_mf.hip, the same bits): its time hardly depends on the tokens
+ * of a tile of 16, k_bf16_gemv_n's is a few us plus so much per token (us,
+ * matrix core / k_bf16_gemv_n: 4096x1024 at 2 tokens 5.5 / 5.3, at 3 5.4 /
+ * 6.2; 256x4096 at 5 10.5 / 9.4, at 6 10.5 / 10.9; 16384x2048 at 5 24.2 /
+ * 23.4, at 6 24.3 / 25.8; 256x7168 at 7 15.9 / 15.5, at 9 15.8 / 19.1;
+ * 64x16384 at 8 31.5 / 29.3, at 9 31.6 / 32.5; 1024x4096 at 48 tokens 11.3 /
+ * 65.9). */
+bool b16n_mf(const B16Geom &g, int rows, int nt)
+{
+    const long long tiles = (long long)((rows + 15) / 16) * ((nt + 15) / 16);
+    return g.tc >= 4 && nt >= (g.ch <= 128 && tiles <= 256 ? 3 : g.ch <= 512 ? 6 : 9);
+}
+
 int b16_dispatch(const B16Geom &g, float *y, const float *x, const uint16_t *W, int rows,
                  int cols, const B16List &ls, hipStream_t st)
 {
@@ -205,6 +219,13 @@ int dsv4_bf16_gemv_n_launch(float *y, const float *x, const uint16_t *W, int row
         DSV4_ERR("bf16 gemv_n: unsupported shape %dx%d, %d tokens, or unaligned operands",
                  rows, cols, nt);
         return -1;
+    }
+    if (b16n_mf(g, rows, nt)) {
+        Dsv4BatchMf b;
+        b.fmt = 2; b.y = y; b.x = x; b.W = W;
+        b.rows = rows; b.cols = cols; b.nt = nt; b.tc = g.tc;
+        const int rc = dsv4_batch_mf_launch(b, st);
+        if (rc <= 0) return rc;
     }
     switch (g.nch) {
     case 1: b16n_launch<1>(g, y, x, W, rows, cols, nt, st); break;

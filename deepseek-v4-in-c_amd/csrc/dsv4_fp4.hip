@@ -235,6 +235,21 @@ void f4n_launch(float *y, const float *x, const uint8_t *W, const uint8_t *S, in
                        blk_r, blk_c, nt, tbx);
 }
 
+/* From how many tokens the batch runs on the f32 matrix core
+ * (dsv4_batch_mf.hip, the same bits): its time hardly depends on the tokens
+ * of a tile of 16, k_fp4_gemv_n's grows with each (us, matrix core /
+ * k_fp4_gemv_n: 7168x2048 at 3 tokens 10.6 / 9.1, at 4 10.5 / 11.0;
+ * 2048x7168 at 3 15.3 / 15.3, at 4 15.4 / 19.1, at 24 16.4 / 102; 512x16384
+ * at 4 29.4 / 27.5, at 5 29.5 / 34.0; 64x7168 at 4 14.7 / 12.6, at 5 14.8 /
+ * 15.5; 64x2048 at 6 6.8 / 6.8; 8192x8192 at 2 32.8 / 44.8, at 64 109 /
+ * 1242). */
+bool f4n_mf(int rows, int cols, int nt)
+{
+    if (cols <= 2048 && rows < 1024) return nt >= 7;
+    if (rows < 1024) return nt >= 5;
+    return nt >= (rows >= 8192 && cols >= 8192 ? 2 : 4);
+}
+
 } // namespace
 
 int dsv4_fp4_gemv_n_launch(float *y, const float *x, const uint8_t *W, const uint8_t *S,
@@ -249,6 +264,14 @@ int dsv4_fp4_gemv_n_launch(float *y, const float *x, const uint8_t *W, const uin
     }
     const int sc = (cols + blk_c - 1) / blk_c;
     const int ch = cols >> 5;
+    if (f4n_mf(rows, cols, nt)) {
+        Dsv4BatchMf b;
+        b.fmt = 3; b.y = y; b.x = x; b.W = W; b.S = S;
+        b.rows = rows; b.cols = cols; b.nt = nt;
+        b.tc = 64; b.sc = sc; b.blk_r = blk_r; b.blk_c = blk_c;
+        const int rc = dsv4_batch_mf_launch(b, st);
+        if (rc <= 0) return rc;
+    }
     if (ch <= 64)       f4n_launch<1>(y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st);
     else if (ch <= 128) f4n_launch<2>(y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st);
     else if (ch <= 256) f4n_launch<4>(y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st);

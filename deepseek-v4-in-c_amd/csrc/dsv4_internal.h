@@ -128,6 +128,24 @@ int dsv4_bf16_gemv_launch(float *y, const float *x, const uint16_t *W, int rows,
 int dsv4_bf16_gemv_n_launch(float *y, const float *x, const uint16_t *W, int rows, int cols,
                             int nt, hipStream_t st);
 
+/* The batched GEMVs on the f32 matrix core (dsv4_batch_mf.hip): fmt 0 FP8
+ * with E8M0 scales, 1 FP8 with fp32 scales, 2 BF16, 3 MXFP4; tc the slots
+ * per row of that format's single-token GEMV, whose bits every (row, token)
+ * gets. 0; 1 where it does not take the shape; -1 on a launch failure. */
+struct Dsv4BatchMf {
+    int fmt = 0;
+    float *y = nullptr;
+    const float *x = nullptr;
+    const void *W = nullptr, *S = nullptr;
+    int rows = 0, cols = 0, nt = 0, tc = 0, sc = 0, blk_r = 0, blk_c = 0;
+    int slots = 0;                             /* per wave; 0: the rule's     */
+    /* split > 1: that many workgroups per tile, their sums of 64 (or, with
+     * fewer, of their own) slots in part and a second launch that joins them */
+    int split = 1;
+    float *part = nullptr;
+};
+int dsv4_batch_mf_launch(const Dsv4BatchMf &b, hipStream_t st);
+
 /* Greedy argmax (the first index of the maximum, dsv4_run.c:471-472) over
  * d_v[n] into d_out[0]; scratch of dsv4_argmax_scratch_bytes. 0 / -1. */
 size_t dsv4_argmax_scratch_bytes(void);
