@@ -1007,19 +1007,22 @@ int dsv4_gpu_moe_fp4_n(float *out, const float *x, int layer, const int *idx,
     const size_t oo = s.add((size_t)nt * hidden * sizeof(float));
     size_t end;
     if (stage_push(s, &end) != 0) return -1;
-    /* With the routing in hand: when the batch's (token, k) pairs barely
-     * share experts (distinct experts above 9 in 10 pairs), reading each
-     * expert once saves next to nothing and the batched passes' per-unit
-     * staging costs more (4 tokens, 31.1 of 32 pairs distinct: 167.1 us
-     * batched against 152.5 us token by token), so the tokens go one by one
-     * through the single-token kernels. Both give every token the same bits.
-     * DSV4_GPU_MOEN_TOKENWISE: 1 always token by token, 0 never. */
+    /* With the routing in hand: two tokens whose (token, k) pairs barely share
+     * experts (distinct experts above 9 in 10 pairs) of C3's size or more go
+     * one by one through the single-token kernels, whose 2 x 8 experts take
+     * 76.1 us at 7168 x 2048 against 79.1 batched. Smaller experts and more
+     * tokens are faster batched with every expert distinct (us, batched /
+     * token by token: 7168 x 2048 top 8, 3 tokens 109.8 / 115.4, 4 tokens
+     * 143.9 / 153.9; 4096 x 2048 top 6, 2 tokens 47.4 / 60.2). Both give
+     * every token the same bits. DSV4_GPU_MOEN_TOKENWISE: 1 always token by
+     * token, 0 never. */
     int tokenwise = moen_tokenwise_env();
     if (tokenwise < 0) {
         std::vector<int> seen(idx, idx + (size_t)nt * topk);
         std::sort(seen.begin(), seen.end());
         const size_t distinct = std::unique(seen.begin(), seen.end()) - seen.begin();
-        tokenwise = nt > 1 && 10 * distinct > 9 * (size_t)nt * topk;
+        tokenwise = nt == 2 && (size_t)hidden * inter >= (size_t)7168 * 2048 &&
+                    10 * distinct > 9 * (size_t)nt * topk;
     }
     if (tokenwise) {
         for (int t = 0; t < nt; t++)

@@ -981,10 +981,9 @@ k_mc2_fused(float *__restrict__ out, uint16_t *__restrict__ ht, const float *__r
 /* ------------------------------------------------------- batched (prefill)
  *
  * The routed half of the reference's moe_n (dsv4_layer.c:714-855) for nt
- * tokens. The batch's (token, k) pairs ask for the distinct experts in
- * first-request order; each distinct expert streams its weights once, for
- * every pair routed to it (the reference's union, :728-739, and
- * run_expert_n, :681-703). Per pair the products are the staged form's
+ * tokens. The distinct experts the batch's (token, k) pairs ask for are
+ * listed, and each streams its weights once, for every pair routed to it (the
+ * reference's union, :728-739, and run_expert_n, :681-703). Per pair the products are the staged form's
  * (k_mc2_gate_up / k_mc2_down), column for column: the matrix core computes
  * each result column from its own B column, so a pair sitting in columns
  * 3j..3j+2 of a 16-column tile gets the bits it gets in columns 0..2 alone.
@@ -992,160 +991,156 @@ k_mc2_fused(float *__restrict__ out, uint16_t *__restrict__ ht, const float *__r
  * k-ordered combine are the single-token ones, so every token's output row
  * is bit-identical to the single-token call on that token.
  *
- * LAUNCHES: k_mn_split (x -> bf16 term planes, every token), k_mn_route (one
- * workgroup: slots, per-slot pair lists), k_mn_pass<GATE> (h of every pair),
- * k_mn_pass<DOWN> (acc_k of every pair), k_mn_combine (the k-ordered sum). */
+ * LAUNCHES: k_mn_prepare (x -> bf16 term planes, every token; slots and
+ * per-slot pair lists), k_mn_pass<GATE> (h of every pair), k_mn_pass<DOWN>
+ * (acc_k of every pair), k_mn_combine (the k-ordered sum). */
 constexpr int MN_TOK = 5;                          /* pairs per 16-column B tile  */
 constexpr int MN_BROWS = MN_TOK * MC_NT;           /* B term rows per tile (15)   */
 constexpr int MN_BP = 512 + 8;                     /* LDS pitch of a term row     */
 constexpr int MN_BBUF = MN_BROWS * MN_BP;          /* bf16 per B buffer           */
-constexpr int MN_NL = (16 * 64) / 256;             /* 16-byte B pieces per thread */
 constexpr int MN_PMAX = 4096;                      /* pairs per call              */
 
 /* Slot s: expert eid[s] (-1 for ids outside the table: its pairs give NaN,
  * as the single-token call does), its pairs plist[off[s] .. off[s] + cnt[s])
- * in pair order (pair p = token * topk + k). */
+ * (pair p = token * topk + k). */
 struct MnRoute {
     int n_uniq, n_pairs, pad[62];
     int eid[MN_PMAX], off[MN_PMAX], cnt[MN_PMAX], plist[MN_PMAX];
 };
 
-__global__ void __launch_bounds__(256)
-k_mn_split(uint16_t *__restrict__ xt, const float *__restrict__ x, int nt, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nt * n) return;
-    const int t = i / n, c = i - t * n;
-    uint32_t tt[MC_NT];
-    bf16_terms(x[i], tt);
-#pragma unroll
-    for (int q = 0; q < MC_NT; q++) xt[((size_t)t * MC_NT + q) * n + c] = (uint16_t)tt[q];
-}
-
-/* One workgroup of 1024. Pair p's key is its expert id (-1 outside the
- * table); its rank is the number of earlier pairs with the same key; rank 0
- * marks the key's first request, and the firsts in pair order number the
- * slots. A pair's place in plist is (pairs of earlier slots) + its rank. */
+/* What the passes need, in one launch of 1024-thread workgroups: workgroup 0
+ * routes, the others split x into its bf16 term planes, four elements per
+ * thread.
+ *
+ * The route. Pair p's key is its expert id (-1 outside the table). The keys
+ * go into a table in LDS (entry id modulo its size, then linear probing; at
+ * least twice the pairs), a pair's rank is its key's count when it arrives,
+ * and one scan over the table numbers the used entries (the slots) and gives
+ * their offsets in plist. The order of an expert's pairs is not the same on
+ * every run; no result depends on it, since a pair has its own columns and
+ * its own place in the results. 5.6 us for 512 pairs and 64 rows of x, against
+ * 32 + 5.4 as two launches with a thread per pair that walked all pairs. */
 __global__ void __launch_bounds__(1024)
-k_mn_route(MnRoute *__restrict__ rt, const int *__restrict__ idx, int np, int n_table)
+k_mn_prepare(MnRoute *__restrict__ rt, const int *__restrict__ idx, int np, int n_table,
+             uint16_t *__restrict__ xt, const float *__restrict__ x, int nt, int n)
 {
-    constexpr int RND = MN_PMAX / 1024;
-    __shared__ int key[MN_PMAX];
-    __shared__ int slot[MN_PMAX];
-    __shared__ int wcnt[RND * 16];
-    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int tid = threadIdx.x, lane = tid & 63;
+    if (blockIdx.x > 0) {
+        const long long i = ((long long)(blockIdx.x - 1) * 1024 + tid) * 4;
+        if (i >= (long long)nt * n) return;
+        const int t = (int)(i / n), c = (int)(i - (long long)t * n);       /* n % 4 == 0 */
+        const f32x4 v = ldf4(x + i);
+        const float vv[4] = {v.x, v.y, v.z, v.w};
+        uint16_t q[MC_NT][4];
 #pragma unroll
-    for (int r = 0; r < RND; r++) {
-        const int p = r * 1024 + tid;
-        if (p < np) {
-            const int e = idx[p];
-            key[p] = (e >= 0 && e < n_table) ? e : -1;
+        for (int e = 0; e < 4; e++) {
+            uint32_t tt[MC_NT];
+            bf16_terms(vv[e], tt);
+#pragma unroll
+            for (int k = 0; k < MC_NT; k++) q[k][e] = (uint16_t)tt[k];
         }
-    }
-    __syncthreads();
-    int q0[RND], rk[RND];
-    unsigned long long bal[RND];
 #pragma unroll
-    for (int r = 0; r < RND; r++) {
-        const int p = r * 1024 + tid;
-        int f = p, c = 0;
-        if (p < np) {
-            const int kp = key[p];
-            for (int q = 0; q < p; q++)
-                if (key[q] == kp) {
-                    if (c == 0) f = q;
-                    c++;
-                }
+        for (int k = 0; k < MC_NT; k++) {
+            uint2 o;
+            o.x = q[k][0] | (uint32_t)q[k][1] << 16;
+            o.y = q[k][2] | (uint32_t)q[k][3] << 16;
+            *reinterpret_cast<uint2 *>(xt + ((size_t)t * MC_NT + k) * n + c) = o;
         }
-        q0[r] = f;
-        rk[r] = c;
-        bal[r] = __ballot(p < np && c == 0);
-        if (lane == 0) wcnt[r * 16 + w] = __popcll(bal[r]);
+        return;
     }
-    __syncthreads();
-    int nu = 0;
-    for (int i = 0; i < RND * 16; i++) nu += wcnt[i];
+    constexpr int RND = MN_PMAX / 1024, TMAX = 2 * MN_PMAX;
+    __shared__ int kt[TMAX];                      /* key, -2: unused          */
+    __shared__ uint32_t ct[TMAX];                 /* its count, then offset   */
+    __shared__ uint32_t wsum[16];
+    const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    int ts = 1024;                                /* entries                  */
+    while (ts < 2 * np) ts *= 2;
+    int key[RND], pos[RND], rank[RND];
 #pragma unroll
     for (int r = 0; r < RND; r++) {
         const int p = r * 1024 + tid;
-        if (p < np && rk[r] == 0) {
-            int base = 0;
-            for (int i = 0; i < r * 16 + w; i++) base += wcnt[i];
-            slot[p] = base + __popcll(bal[r] & ((1ull << lane) - 1ull));
-        }
+        const int e = p < np ? idx[p] : -1;
+        key[r] = (e >= 0 && e < n_table) ? e : -1;
     }
-    __syncthreads();
-    int sl[RND];
-#pragma unroll
-    for (int r = 0; r < RND; r++) {
-        const int p = r * 1024 + tid;
-        sl[r] = p < np ? slot[q0[r]] : 0;
+    for (int i = tid; i < ts; i += 1024) {
+        kt[i] = -2;
+        ct[i] = 0u;
     }
     __syncthreads();
 #pragma unroll
     for (int r = 0; r < RND; r++) {
-        const int p = r * 1024 + tid;
-        if (p < np) slot[p] = sl[r];
+        if (r * 1024 + tid >= np) continue;
+        int h = key[r] & (ts - 1);
+        for (;;) {                                /* an unused entry exists: ts >= 2 np */
+            const int old = atomicCAS(&kt[h], -2, key[r]);
+            if (old == -2 || old == key[r]) break;
+            h = (h + 1) & (ts - 1);
+        }
+        pos[r] = h;
+        rank[r] = (int)atomicAdd(&ct[h], 1u);
+    }
+    __syncthreads();
+    /* exclusive scan over the entries of (used, its pairs) as (high, low) 16
+     * bits: both stay at most MN_PMAX */
+    const int per = ts >> 10;                     /* entries per thread, <= 8 */
+    uint32_t sum = 0;
+    for (int i = 0; i < per; i++) {
+        const uint32_t c = ct[tid * per + i];
+        sum += c ? (1u << 16) + c : 0u;
+    }
+    uint32_t inc = sum;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const uint32_t v = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += v;
+    }
+    if (lane == 63) wsum[w] = inc;
+    __syncthreads();
+    uint32_t at = inc - sum, total = 0;
+    for (int i = 0; i < 16; i++) {
+        if (i < w) at += wsum[i];
+        total += wsum[i];
+    }
+    for (int i = 0; i < per; i++) {
+        const uint32_t c = ct[tid * per + i];
+        if (!c) continue;
+        const int s = (int)(at >> 16);
+        ct[tid * per + i] = at & 0xFFFFu;
+        rt->off[s] = (int)(at & 0xFFFFu);
+        rt->cnt[s] = (int)c;
+        rt->eid[s] = kt[tid * per + i];
+        at += (1u << 16) + c;
     }
     __syncthreads();
 #pragma unroll
-    for (int r = 0; r < RND; r++) {
-        const int p = r * 1024 + tid;
-        if (p >= np) continue;
-        const int sp = sl[r];
-        int less = 0, same = 0;
-        for (int q = 0; q < np; q++) {
-            const int sq = slot[q];
-            less += sq < sp;
-            same += sq == sp;
-        }
-        rt->plist[less + rk[r]] = p;
-        if (rk[r] == 0) {
-            rt->off[sp] = less;
-            rt->cnt[sp] = same;
-            rt->eid[sp] = key[p];
-        }
-    }
+    for (int r = 0; r < RND; r++)
+        if (r * 1024 + tid < np) rt->plist[(int)ct[pos[r]] + rank[r]] = r * 1024 + tid;
     if (tid == 0) {
-        rt->n_uniq = nu;
+        rt->n_uniq = (int)(total >> 16);
         rt->n_pairs = np;
     }
 }
 
-/* The B terms of unit u for a pass's nb pairs: term row (j MC_NT + c) is
- * plane c of source row prow[j] (src [row][MC_NT][K]), 512 elements from
- * 512 u. Requested by every thread (rows past the pass read prow[0], rows
- * past the tile too: no branch before the loads), stored as zeros past nb. */
-__device__ __forceinline__ void mn_bload(u32x4 *v, const uint16_t *src, const int *prow,
-                                         int nb, int K, int u)
+typedef __attribute__((address_space(3))) void lds_void;
+
+/* One term row of one unit, 1 KiB at byte `at` of src (src_bytes long), to
+ * dst in LDS without passing through registers: lane l's 16 bytes at dst +
+ * 16 l. */
+__device__ __forceinline__ void mn_copy_row(const uint16_t *src, uint32_t src_bytes,
+                                            uint16_t *dst, uint32_t at)
 {
-#pragma unroll
-    for (int m = 0; m < MN_NL; m++) {
-        const int i = (int)threadIdx.x + 256 * m;
-        const int row = i >> 6, piece = i & 63;
-        const int j = row / MC_NT, c = row - j * MC_NT;
-        const int pr = j < nb ? prow[j] : prow[0];
-        v[m] = *(const DSV4_GLOBAL u32x4 *)(src + ((size_t)pr * MC_NT + c) * K + 512 * u +
-                                            8 * piece);
-    }
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(src), 0, (int)src_bytes,
+                                          0x00020000),
+        (lds_void *)dst, 16, 16 * (int)(threadIdx.x & 63), (int)at, 0, 0);
 }
 
-__device__ __forceinline__ void mn_bstore(uint16_t *bb, const u32x4 *v, int nb)
-{
-#pragma unroll
-    for (int m = 0; m < MN_NL; m++) {
-        const int i = (int)threadIdx.x + 256 * m;
-        const int row = i >> 6, piece = i & 63;
-        if (row < MN_BROWS)
-            *reinterpret_cast<u32x4 *>(bb + row * MN_BP + 8 * piece) =
-                row / MC_NT < nb ? v[m] : u32x4{0u, 0u, 0u, 0u};
-    }
-}
-
-/* m2_mac with the B tile of a pass: column r reads term row r (15 rows; the
- * unused column 15 repeats row 14). Same steps, same accumulators. */
-__device__ __forceinline__ void mn_mac(v4f *acc, const unsigned char *buf, const uint16_t *bb,
-                                       int lane, bool live)
+/* m2_mac with a pass's CT column tiles of five pairs: column r of tile t
+ * reads term row 15 t + r (the unused column 15 repeats row 14). Each tile's
+ * steps and accumulators are m2_mac's. */
+template <int CT>
+__device__ __forceinline__ void mn_mac(v4f (*acc)[2], const unsigned char *buf,
+                                       const uint16_t *bb, int lane, bool live)
 {
     const int r = lane & 15, g = lane >> 4;
     const u32x4 sv = *reinterpret_cast<const u32x4 *>(buf + M2_SOFF + r * 16);
@@ -1156,15 +1151,22 @@ __device__ __forceinline__ void mn_mac(v4f *acc, const unsigned char *buf, const
         const u32x4 a = *reinterpret_cast<const u32x4 *>(buf + r * M2_WP + 64 * qb + 16 * g);
         const float sc = live ? dec_e8m0((sw[qb] >> (8 * g)) & 0xFFu) : 0.0f;
         const uint32_t d[4] = {a.x, a.y, a.z, a.w};
-        v8bf b[4];
+        v8bf b[CT][4];
 #pragma unroll
-        for (int m = 0; m < 4; m++)
-            b[m] = __builtin_bit_cast(v8bf, *reinterpret_cast<const u32x4 *>(
-                                                bl + 128 * qb + 32 * g + 8 * m));
+        for (int t = 0; t < CT; t++)
 #pragma unroll
-        for (int m = 0; m < 4; m++)
-            acc[qb & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fp4x8_bf16(d[m], sc), b[m],
-                                                                   acc[qb & 1], 0, 0, 0);
+            for (int m = 0; m < 4; m++)
+                b[t][m] = __builtin_bit_cast(
+                    v8bf, *reinterpret_cast<const u32x4 *>(bl + t * MN_BROWS * MN_BP + 128 * qb +
+                                                           32 * g + 8 * m));
+#pragma unroll
+        for (int m = 0; m < 4; m++) {
+            const v8bf w = fp4x8_bf16(d[m], sc);
+#pragma unroll
+            for (int t = 0; t < CT; t++)
+                acc[t][qb & 1] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, b[t][m],
+                                                                         acc[t][qb & 1], 0, 0, 0);
+        }
     }
 }
 
@@ -1184,11 +1186,87 @@ __device__ __forceinline__ v4f term_sum_at(const v4f &d, int lane, int c0)
     return s;
 }
 
-__device__ __forceinline__ void mn_wave_sync()
+/* One pass's units for one wave: res[t] = column tile t's sums of the wave's
+ * 16 rows (weights at base, scales at sb, nu units) with the pass's nb pairs'
+ * terms (rows prow[j] of src).
+ *
+ * The terms of a unit (3 nb rows of 1 KiB) are copied into one of two LDS
+ * buffers by direct-to-LDS loads, RPW of them per wave (row w, w + 4, ...;
+ * past the last row the last again), one unit ahead; the weights D units
+ * ahead into registers, then through the wave's own buffer. Per unit: the
+ * weights into that buffer, the wait for the wave's term copies (the next
+ * weight unit, requested after them, stays in flight), one barrier (every
+ * wave's copies have arrived, and every wave is done with the other buffer),
+ * the next copies and weights requested, the unit's products.
+ *
+ * What bounds it: the weight stream. C3's expert shape, 64 tokens of 256
+ * experts, us per call: 1155 with all 16 term rows of a tile brought through
+ * registers per unit whatever the pass's pairs, 967 with this; 914 with the
+ * terms left out altogether and 864 (6.1 TB/s) with the products left out
+ * too. D = 3 or 4 weight units in flight measured the same (966, 993). */
+template <int D, int NU, int CT, int RPW>
+__device__ __forceinline__ void mn_units(v4f *res, const uint16_t *src, uint32_t src_bytes,
+                                         const int *prow, int nb, int K, const uint8_t *base,
+                                         const uint8_t *sb, int nu, uint16_t *bbuf,
+                                         unsigned char *buf)
 {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    constexpr int BBUF = CT * MN_BROWS * MN_BP;
+    const int lane = threadIdx.x & 63;
+    const int w = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+    const int nsb = K >> 5;
+    const size_t rowb = (size_t)K >> 1;
+    const int nup = NU > 0 ? NU : ((nu + D - 1) / D) * D;   /* units run, dead included */
+    uint32_t from[RPW];
+    int to[RPW];
+#pragma unroll
+    for (int i = 0; i < RPW; i++) {
+        const int row = min(w + 4 * i, nb * MC_NT - 1);
+        const int j = row / MC_NT, c = row - j * MC_NT;
+        from[i] = (uint32_t)(__builtin_amdgcn_readfirstlane(prow[j]) * MC_NT + c) * (uint32_t)K * 2u;
+        to[i] = row * MN_BP;
+    }
+    auto terms = [&](int u) {                              /* unit u's, clamped to the last */
+        uint16_t *bb = bbuf + (u & 1) * BBUF;
+        const uint32_t k0 = 1024u * (uint32_t)min(u, nu - 1);
+#pragma unroll
+        for (int i = 0; i < RPW; i++) mn_copy_row(src, src_bytes, bb + to[i], from[i] + k0);
+    };
+    M2Unit P[D];
+    terms(0);
+    __builtin_amdgcn_sched_barrier(0);
+    m2_prologue<D>(P, base, rowb, sb, nsb, nu, lane);
+    __builtin_amdgcn_sched_barrier(0);
+    v4f acc[CT][2];
+#pragma unroll
+    for (int t = 0; t < CT; t++) acc[t][0] = acc[t][1] = v4f{0.f, 0.f, 0.f, 0.f};
+    auto unit = [&](int u, M2Unit &slot) {
+        m2_stage(buf, slot, lane);
+        /* the copies of unit u were requested before the 5 loads of weight
+         * unit u + D - 1 (the prologue's: before all of them); past the last
+         * unit nothing follows them */
+        if (NU == 0 || u + D - 1 < nup) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+        else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+        if (NU == 0 || u + 1 < nup) terms(u + 1);
+        __builtin_amdgcn_sched_barrier(0);
+        if (NU == 0 || u + D < nup)
+            m2_load(slot, base, rowb, sb, nsb, min(u + D, nu - 1), lane);
+        __builtin_amdgcn_sched_barrier(0);
+        mn_mac<CT>(acc, buf, bbuf + (u & 1) * BBUF, lane, u < nu);
+    };
+    if constexpr (NU > 0) {
+#pragma unroll
+        for (int u = 0; u < NU; u++) unit(u, P[u % D]);
+    } else {
+        for (int u0 = 0; u0 < nup; u0 += D) {
+#pragma unroll
+            for (int j = 0; j < D; j++) unit(u0 + j, P[j]);
+        }
+        /* the requests past the end land before their buffers are reused */
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+#pragma unroll
+    for (int t = 0; t < CT; t++) res[t] = acc[t][0] + acc[t][1];
 }
 
 /* One pass kernel for both halves; workgroup (row block, slot), 4 waves, a
@@ -1198,23 +1276,21 @@ __device__ __forceinline__ void mn_wave_sync()
  *         SwiGLU, h terms into dst = ht [pair][MC_NT][inter];
  *   DOWN: rows blockIdx.x * 64 + 16 w of w2, B = the pairs' h terms (src =
  *         ht); acc_k into dst = accp [pair][hidden].
- * The slot's pairs run in passes of MN_TOK. Per unit: each wave stages its
- * weight unit (requested D units earlier) in its own buffer, requests the
- * next unit's B and the weight unit D ahead (B first: the end-of-unit wait
- * for B then leaves that weight unit in flight), runs the unit, stores the
- * next B into the other buffer, and the workgroup meets at one barrier. NU >
- * 0: the unit count, every unit live (k_mc2_*'s NU > 0 forms); NU == 0: a
+ * The slot's pairs run in passes of up to CTM column tiles of MN_TOK; a pass
+ * takes the tiles and the term copies that its pairs need (mn_units). NU > 0:
+ * the unit count, every unit live (k_mc2_*'s NU > 0 forms); NU == 0: a
  * run-time count padded to a multiple of D with dead units, as m2_tile's
  * run-time form pads (D must then equal the single-token form's, 3). */
-template <int D, int NU, bool GATE>
+template <int D, int NU, bool GATE, int CTM>
 __global__ void __launch_bounds__(256)
-k_mn_pass(void *__restrict__ dst, const uint16_t *__restrict__ src,
+k_mn_pass(void *__restrict__ dst, const uint16_t *__restrict__ src, uint32_t src_bytes,
           const MnRoute *__restrict__ rt, const Dsv4ExpertDev *__restrict__ table,
           int topk, int hidden, int inter, float limit)
 {
     extern __shared__ __attribute__((aligned(16))) unsigned char mnlds[];
-    __shared__ float red[2][2][MN_TOK][16];             /* GATE: [tile][mat][pair][row] */
-    __shared__ int prow[MN_TOK], pidx[MN_TOK];
+    constexpr int TOK = CTM * MN_TOK;
+    __shared__ float red[2][2][TOK][16];                /* GATE: [tile][mat][pair][row] */
+    __shared__ int prow[TOK], pidx[TOK];
     const int sl = blockIdx.y;
     if (sl >= rt->n_uniq) return;                       /* the whole workgroup */
     const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
@@ -1235,57 +1311,40 @@ k_mn_pass(void *__restrict__ dst, const uint16_t *__restrict__ src,
     const int nsb = K >> 5;
     const size_t rowb = (size_t)K >> 1;
     const int nu = NU > 0 ? NU : (int)(rowb / M2_UB);
-    const int nup = NU > 0 ? NU : ((nu + D - 1) / D) * D;   /* units run, dead included */
     const int mat = GATE ? (w & 1) : 0, tile = GATE ? (w >> 1) : w;
     const int o0 = GATE ? blockIdx.x * 32 + 16 * tile : blockIdx.x * 64 + 16 * w;
     const uint8_t *base = (GATE ? (mat ? E.w3 : E.w1) : E.w2) + (size_t)o0 * rowb;
     const uint8_t *sb = (GATE ? (mat ? E.s3 : E.s1) : E.s2) + (size_t)o0 * nsb;
-    uint16_t *bbuf = (uint16_t *)mnlds;                             /* [2][MN_BBUF] */
-    unsigned char *buf = mnlds + (size_t)2 * MN_BBUF * 2 + (size_t)w * M2_WBUF;
+    uint16_t *bbuf = (uint16_t *)mnlds;                    /* [2][CTM][MN_BBUF] */
+    unsigned char *buf = mnlds + (size_t)2 * CTM * MN_BBUF * 2 + (size_t)w * M2_WBUF;
     const int r = lane & 15, g = lane >> 4;
 
-    for (int p0 = 0; p0 < cnt; p0 += MN_TOK) {
-        const int nb = min(MN_TOK, cnt - p0);
+    for (int p0 = 0; p0 < cnt; p0 += TOK) {
+        const int nb = min(TOK, cnt - p0);
         __syncthreads();                                /* the last pass's epilogue */
-        if (tid < MN_TOK) {
+        if (tid < TOK) {
             const int p = rt->plist[off + p0 + min(tid, nb - 1)];
             pidx[tid] = p;
             prow[tid] = GATE ? p / topk : p;
         }
         __syncthreads();
-        u32x4 bv[MN_NL];
-        M2Unit P[D];
-        mn_bload(bv, src, prow, nb, K, 0);
-        __builtin_amdgcn_sched_barrier(0);
-        m2_prologue<D>(P, base, rowb, sb, nsb, nu, lane);
-        __builtin_amdgcn_sched_barrier(0);
-        mn_bstore(bbuf, bv, nb);
-        __syncthreads();
-        v4f acc[2] = {v4f{0.f, 0.f, 0.f, 0.f}, v4f{0.f, 0.f, 0.f, 0.f}};
-        auto unit = [&](int u, M2Unit &slot) {
-            m2_stage(buf, slot, lane);
-            mn_bload(bv, src, prow, nb, K, min(u + 1, nu - 1));
-            __builtin_amdgcn_sched_barrier(0);
-            if (NU == 0 || u + D < nup)
-                m2_load(slot, base, rowb, sb, nsb, min(u + D, nu - 1), lane);
-            __builtin_amdgcn_sched_barrier(0);
-            mn_wave_sync();
-            mn_mac(acc, buf, bbuf + (u & 1) * MN_BBUF, lane, u < nu);
-            mn_bstore(bbuf + ((u + 1) & 1) * MN_BBUF, bv, nb);
-            __syncthreads();
-        };
-        if constexpr (NU > 0) {
-#pragma unroll
-            for (int u = 0; u < NU; u++) unit(u, P[u % D]);
-        } else {
-            for (int u0 = 0; u0 < nup; u0 += D) {
-#pragma unroll
-                for (int j = 0; j < D; j++) unit(u0 + j, P[j]);
-            }
+        v4f res[CTM];
+#define MN_GO(CT, RPW)                                                                      \
+    mn_units<D, NU, CT, RPW>(res, src, src_bytes, prow, nb, K, base, sb, nu, bbuf, buf)
+        if (nb == 1) MN_GO(1, 1);
+        else if (nb == 2) MN_GO(1, 2);
+        else if (nb <= 4) MN_GO(1, 3);
+        else if (CTM == 1 || nb <= MN_TOK) MN_GO(1, 4);
+        else if constexpr (CTM > 1) {
+            MN_GO(2, 8);
         }
-        const v4f res = acc[0] + acc[1];
+#undef MN_GO
         for (int j = 0; j < nb; j++) {
-            const v4f sj = term_sum_at(res, lane, MC_NT * j);
+            v4f rs = res[0];
+#pragma unroll
+            for (int t = 1; t < CTM; t++)
+                if (j / MN_TOK == t) rs = res[t];
+            const v4f sj = term_sum_at(rs, lane, MC_NT * (j % MN_TOK));
             if (r == 0) {
 #pragma unroll
                 for (int jj = 0; jj < 4; jj++) {
@@ -1329,7 +1388,7 @@ k_mn_combine(float *__restrict__ out, const float *__restrict__ accp,
     out[(size_t)t * hidden + i] = o;
 }
 
-size_t mn_lds() { return (size_t)2 * MN_BBUF * 2 + 4 * M2_WBUF; }
+size_t mn_lds(int ctm) { return (size_t)2 * ctm * MN_BBUF * 2 + 4 * M2_WBUF; }
 
 size_t m2_lds_a(int hidden) { return (size_t)MC_NT * mc_pitch(hidden) * 2 + 4 * M2_WBUF; }
 size_t m2_lds_b(int topk, int inter) { return (size_t)m2_down_waves(topk) * m2_wave_b(inter); }
@@ -1502,7 +1561,7 @@ int dsv4_moe_fp4_n_launch(float *d_out, const float *d_x, const Dsv4ExpertDev *d
     const int form = mc_env("DSV4_GPU_MOE_MC", 2);
     const bool batched = nt > 1 && form == 2 && m2_shape_ok(topk, hidden, inter) &&
                          ((uintptr_t)d_x & 15u) == 0 && (size_t)nt * topk <= MN_PMAX &&
-                         mn_lds() + 8 * 1024 <= dsv4_lds_limit();
+                         mn_lds(1) + 8 * 1024 <= dsv4_lds_limit();
     if (!batched) {
         /* token by token: each token's own call, so its bits by construction */
         for (int t = 0; t < nt; t++)
@@ -1520,32 +1579,45 @@ int dsv4_moe_fp4_n_launch(float *d_out, const float *d_x, const Dsv4ExpertDev *d
     uint16_t *ht = (uint16_t *)p;                       p += a256((size_t)np * MC_NT * inter * 2);
     float *accp = (float *)p;
     const int slots = np < n_table + 1 ? np : n_table + 1;
-    static bool opted = false;
-    if (!opted) {
-        mc_lds_optin(k_mn_pass<2, 14, true>); mc_lds_optin(k_mn_pass<3, 0, true>);
-        mc_lds_optin(k_mn_pass<2, 4, false>); mc_lds_optin(k_mn_pass<3, 0, false>);
-        opted = true;
-    }
-    const size_t lds = mn_lds();
-    hipLaunchKernelGGL(k_mn_split, dim3((nt * hidden + 255) / 256), dim3(256), 0, st, xt, d_x,
-                       nt, hidden);
-    hipLaunchKernelGGL(k_mn_route, dim3(1), dim3(1024), 0, st, rt, d_idx, np, n_table);
+    hipLaunchKernelGGL(k_mn_prepare, dim3(1 + (unsigned)(((long long)nt * hidden / 4 + 1023) / 1024)),
+                       dim3(1024), 0, st, rt, d_idx, np, n_table, xt, d_x, nt, hidden);
     HIP_OK(hipGetLastError(), "moe_n route launch");
     const dim3 ga(inter / 32, slots), gb(hidden / 64, slots);
-    if (hidden / 512 == 14)
-        hipLaunchKernelGGL((k_mn_pass<2, 14, true>), ga, dim3(256), lds, st, (void *)ht, xt, rt,
-                           d_table, topk, hidden, inter, limit);
-    else
-        hipLaunchKernelGGL((k_mn_pass<3, 0, true>), ga, dim3(256), lds, st, (void *)ht, xt, rt,
-                           d_table, topk, hidden, inter, limit);
-    HIP_OK(hipGetLastError(), "moe_n gate/up launch");
-    if (inter / 512 == 4)
-        hipLaunchKernelGGL((k_mn_pass<2, 4, false>), gb, dim3(256), lds, st, (void *)accp, ht,
-                           rt, d_table, topk, hidden, inter, limit);
-    else
-        hipLaunchKernelGGL((k_mn_pass<3, 0, false>), gb, dim3(256), lds, st, (void *)accp, ht,
-                           rt, d_table, topk, hidden, inter, limit);
-    HIP_OK(hipGetLastError(), "moe_n down launch");
+    const uint32_t xb = (uint32_t)((size_t)nt * MC_NT * hidden * 2);
+    const uint32_t hb = (uint32_t)((size_t)np * MC_NT * inter * 2);
+    /* a second column tile per pass where the experts average more than its
+     * five pairs, so that most take one pass over their weights; its LDS (81
+     * against 50 KB) leaves two workgroups per CU instead of three (us, two /
+     * one tile, 7168 x 2048, top 8: 64 tokens of 64 experts 524 / 627, of 16
+     * 461 / 594; 32 tokens of 64 experts 390 / 368, 64 tokens of 256 1165 /
+     * 967; three tiles 571, 470, 443, 1356) */
+    const int ctm = np > 5 * n_table ? 2 : 1;
+    static bool opted = false;
+    if (!opted) {
+        mc_lds_optin(k_mn_pass<2, 14, true, 1>); mc_lds_optin(k_mn_pass<3, 0, true, 1>);
+        mc_lds_optin(k_mn_pass<2, 4, false, 1>); mc_lds_optin(k_mn_pass<3, 0, false, 1>);
+        mc_lds_optin(k_mn_pass<2, 14, true, 2>); mc_lds_optin(k_mn_pass<3, 0, true, 2>);
+        mc_lds_optin(k_mn_pass<2, 4, false, 2>); mc_lds_optin(k_mn_pass<3, 0, false, 2>);
+        opted = true;
+    }
+    auto go = [&](auto kern, dim3 grid, void *dst, const uint16_t *src, uint32_t bytes) {
+        hipLaunchKernelGGL(kern, grid, dim3(256), mn_lds(ctm), st, dst, src, bytes, rt, d_table,
+                           topk, hidden, inter, limit);
+        HIP_OK(hipGetLastError(), "moe_n pass launch");
+        return 0;
+    };
+    if (hidden / 512 == 14
+            ? (ctm == 1 ? go(k_mn_pass<2, 14, true, 1>, ga, ht, xt, xb)
+                        : go(k_mn_pass<2, 14, true, 2>, ga, ht, xt, xb))
+            : (ctm == 1 ? go(k_mn_pass<3, 0, true, 1>, ga, ht, xt, xb)
+                        : go(k_mn_pass<3, 0, true, 2>, ga, ht, xt, xb)))
+        return -1;
+    if (inter / 512 == 4
+            ? (ctm == 1 ? go(k_mn_pass<2, 4, false, 1>, gb, accp, ht, hb)
+                        : go(k_mn_pass<2, 4, false, 2>, gb, accp, ht, hb))
+            : (ctm == 1 ? go(k_mn_pass<3, 0, false, 1>, gb, accp, ht, hb)
+                        : go(k_mn_pass<3, 0, false, 2>, gb, accp, ht, hb)))
+        return -1;
     hipLaunchKernelGGL(k_mn_combine, dim3((hidden + 255) / 256, nt), dim3(256), 0, st, d_out,
                        accp, d_w, topk, hidden);
     HIP_OK(hipGetLastError(), "moe_n combine launch");

@@ -333,8 +333,8 @@ int dsv4_gpu_moe_fp4_d(float *d_out, const float *d_x, int layer,
  * path) on the device: out[t] = dsv4_gpu_moe_fp4 of token t, for nt <=
  * DSV4_MAX_BATCH tokens (x/out [nt][hidden], idx/w [nt][topk], host
  * buffers). As in the reference, the distinct experts the batch asks for are
- * found first (in first-request order) and each one's weights are read once
- * for every (token, k) routed to it; each token's row is bit-identical to
+ * found first and each one's weights are read once for every (token, k)
+ * routed to it; each token's row is bit-identical to
  * dsv4_gpu_moe_fp4 on that token. 0 / -1 (an expert not resident, a shape
  * that does not match, nt out of range). */
 int dsv4_gpu_moe_fp4_n(float *out, const float *x, int layer, const int *idx,
