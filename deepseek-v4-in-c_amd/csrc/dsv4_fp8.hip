@@ -39,7 +39,6 @@
 
 #include <algorithm>
 #include <stdlib.h>
-#include <type_traits>
 
 namespace {
 
@@ -76,11 +75,24 @@ bool fp8_geom(int cols, Fp8Geom *g)
     return true;
 }
 
+/* A scale as it lies in memory, and its value. A load whose result is decoded
+ * where it is needed and not where it is issued does not make the loads
+ * issued before it be waited for there. */
+template <int SF>
+__device__ __forceinline__ uint32_t ld_scale_raw(const void *S, size_t at)
+{
+    if (SF == 0) return ((const uint8_t *)S)[at];
+    return ((const uint32_t *)S)[at];
+}
+template <int SF>
+__device__ __forceinline__ float scale_val(uint32_t raw)
+{
+    return SF == 0 ? dec_e8m0(raw) : __uint_as_float(raw);
+}
 template <int SF>
 __device__ __forceinline__ float ld_scale(const void *S, size_t at)
 {
-    if (SF == 0) return dec_e8m0(((const uint8_t *)S)[at]);
-    return ((const float *)S)[at];
+    return scale_val<SF>(ld_scale_raw<SF>(S, at));
 }
 
 /* Dot of 16 decoded weights with 16 activations; 4 interleaved chains. */
@@ -147,7 +159,7 @@ struct Fp8Groups {
  * the last chunk, and their results are discarded -- so no branch stands
  * between the loads and the waits that count them. */
 template <int NCH, int R, int SF>
-__device__ __forceinline__ void load_step(u32x4 (*wv)[NCH], float *sv, const uint8_t *W,
+__device__ __forceinline__ void load_step(u32x4 (*wv)[NCH], uint32_t *sv, const uint8_t *W,
                                           const void *S, int rbase, int rend, int cols,
                                           int ch, int j, int tc, const int *cb, int sc,
                                           int blk_r)
@@ -163,7 +175,7 @@ __device__ __forceinline__ void load_step(u32x4 (*wv)[NCH], float *sv, const uin
     }
     const int rb = min(rbase, rend - 1) / blk_r;
 #pragma unroll
-    for (int n = 0; n < NCH; n++) sv[n] = ld_scale<SF>(S, (size_t)rb * sc + cb[n]);
+    for (int n = 0; n < NCH; n++) sv[n] = ld_scale_raw<SF>(S, (size_t)rb * sc + cb[n]);
 }
 
 /* One workgroup owns the contiguous rows [row0, row0 + rows_per_wg). It walks
@@ -221,15 +233,24 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
     }
 
     u32x4 wv[R][NCH], wn[R][NCH];
-    float sv[NCH], sn[NCH];
+    uint32_t sv[NCH], sn[NCH];
     if (XL) {
         /* x once per workgroup: the whole workgroup requests all of x (four
          * floats per thread per round, all rounds issued together), then the
          * first step's weights; x lands in LDS and each thread reads its
          * slice from there. Without this, every row group of the workgroup
-         * would fetch the same x from L2. */
+         * would fetch the same x from L2.
+         *
+         * What is meant to overlap is x's way through LDS (and the norm) with
+         * the first weights' latency, so nothing here may wait for those: the
+         * scales stay raw, no branch stands between the loads and the waits
+         * that count them (lanes past x's end load and store its last
+         * piece), and the rounds are the row's own (XL 1: a row of at most 64
+         * threads, XL 2: any). With the scales decoded where loaded and four
+         * times the rounds, x was stored only once the weights had arrived
+         * (24576x1536 9.26 us, now 8.54). */
         float *xs = part + (size_t)(tc > 64 ? tc / 64 : 0) * rows_per_wg;
-        constexpr int XR = 4 * NCH;                    /* rounds: cols <= 1024 XR */
+        constexpr int XR = XL == 1 ? NCH : 4 * NCH;    /* rounds: cols <= 1024 XR */
         f32x4 xv[XR], nv[NQ ? XR : 1];
         const int nq = cols >> 2;
         /* (NQ: the norm's weights with x, ahead of the weights' requests, and
@@ -242,17 +263,13 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
             if (NQ) nv[q] = ldf4(nq_w + i);
         }
         __builtin_amdgcn_sched_barrier(0);
-        if (nsteps > 0)
-            load_step<NCH, R, SF>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb, sc,
-                                  blk_r);
+        load_step<NCH, R, SF>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb, sc, blk_r);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int q = 0; q < XR; q++) {
-            const int i = q * (int)blockDim.x + tid;
-            if (i < nq) {
-                *reinterpret_cast<f32x4 *>(xs + 4 * i) = xv[q];
-                if (NQ) *reinterpret_cast<f32x4 *>(xw + 4 * i) = nv[q];
-            }
+            const int i = 4 * min(q * (int)blockDim.x + tid, nq - 1);
+            *reinterpret_cast<f32x4 *>(xs + i) = xv[q];
+            if (NQ) *reinterpret_cast<f32x4 *>(xw + i) = nv[q];
         }
         __syncthreads();
         if (NQ) {
@@ -294,9 +311,7 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
                 xr[n][q * 4 + 2] = v.z; xr[n][q * 4 + 3] = v.w;
             }
         }
-        if (nsteps > 0)
-            load_step<NCH, R, SF>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb, sc,
-                                  blk_r);
+        load_step<NCH, R, SF>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb, sc, blk_r);
     }
 
     for (int step = 0; step < nsteps; ++step) {
@@ -311,7 +326,7 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
             float a = 0.0f;
 #pragma unroll
             for (int n = 0; n < NCH; n++) {
-                const float d = fmaf(dot16(wv[i][n], xr[n]), sv[n], a);
+                const float d = fmaf(dot16(wv[i][n], xr[n]), scale_val<SF>(sv[n]), a);
                 a = act[n] ? d : a;
             }
             acc[i] = a;
@@ -547,10 +562,15 @@ void launch_gemv(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
         if (!opted) {
             (void)dsv4_lds_optin((const void *)k_fp8_gemv<NCH, R, SF, PF, 1>,
                                  dsv4_lds_limit(), "fp8 gemv");
+            (void)dsv4_lds_optin((const void *)k_fp8_gemv<NCH, R, SF, PF, 2>,
+                                 dsv4_lds_limit(), "fp8 gemv");
             opted = true;
         }
     }
-    if (xl)
+    if (xl && g.tc > 64)
+        hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 2>), dim3(grid, gp.n), dim3(g.wg), lds,
+                           st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
+    else if (xl)
         hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 1>), dim3(grid, gp.n), dim3(g.wg), lds,
                            st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
     else
@@ -1269,7 +1289,11 @@ int dsv4_qproj_launch(const float *qr, int cols, const float *nw, float eps, int
      * with no prefetch in the x launch measured slower (78.7), so that
      * launch keeps two rows with prefetch. */
     const int qrr = env_int("DSV4_GPU_QPROJ_R", 4) >= 4 && blk_r % 4 == 0 ? 4 : 2;
-    const Fp8Plan pf = fp8_plan(g, qrr, rm, cols, v.wpc, nf);
+    /* each matrix the grid it would have alone, not a share of one: each
+     * workgroup's norm stands between its first weights and the rest, and
+     * the more of them there are the more weights are in flight meanwhile
+     * (the CSA step above 75.6 -> 73.8 us). */
+    const Fp8Plan pf = fp8_plan(g, qrr, rm, cols, v.wpc, 1);
     /* the combinations built: x through LDS (cols <= 2048), 1 or 2 chunks
      * per thread, 2 or 4 rows per step, no prefetch (wq_b's rows), 256
      * threads */

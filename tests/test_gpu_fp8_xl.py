@@ -1,0 +1,43 @@
+"""The single-token FP8 GEMV with x through LDS (csrc/dsv4_fp8.hip) at the
+edges of its rounds of 1024 columns: rows of 1 to 64 threads and of 65 to 256,
+x that ends inside a round, and rows that end inside a workgroup's step. x
+straight from memory and through LDS are the same arithmetic, so their bits
+are equal; against 64 bits the error is that of a sum of `cols` products in
+f32, bounded by cols * 2^-24 of the sum of their magnitudes."""
+import ctypes
+
+import numpy as np
+import pytest
+
+import common
+
+pytestmark = pytest.mark.gpu
+
+_KEEP = []          # resident matrices are keyed by host address
+
+
+@pytest.mark.parametrize("scales", ["e8m0", "f32"])
+@pytest.mark.parametrize("rows,cols", [
+    (1, 16), (5, 48), (700, 512), (130, 1008), (64, 1024), (67, 1040), (1025, 1536),
+    (259, 2032), (2100, 2048), (33, 2064), (70, 4096), (37, 8192), (35, 16368), (300, 16384)])
+def test_x_through_lds(gpu, dsv4, monkeypatch, rows, cols, scales):
+    rng = np.random.default_rng(rows * 31 + cols)
+    W = common.fp8_codes(rng, (rows, cols))
+    Sf, Se = common.fp8_scales(rng, rows, cols)
+    S = Se if scales == "e8m0" else Sf
+    _KEEP.append((W, S))
+    m = dsv4.qmat(W, S)
+    up = gpu.dsv4_gpu_upload if scales == "e8m0" else gpu.dsv4_gpu_upload_f32s
+    assert up(ctypes.byref(m)) == 0
+    x = rng.standard_normal(cols, dtype=np.float32)
+    got = {}
+    for xl in ("0", "1"):
+        for r in ("1", "4"):
+            monkeypatch.setenv("DSV4_GPU_FP8_XL", xl)
+            monkeypatch.setenv("DSV4_GPU_FP8_R", r)
+            got[xl, r] = dsv4.mmq(m, x).copy()
+    for y in got.values():
+        assert common.bits_equal(y, got["0", "1"])
+    s = np.repeat(np.repeat(Sf.astype(np.float64), 128, 0)[:rows], 128, 1)[:, :cols]
+    p = common.e4m3_table()[W].astype(np.float64) * s * x
+    assert np.all(np.abs(got["1", "1"] - p.sum(1)) <= cols * 2.0 ** -24 * np.abs(p).sum(1))
