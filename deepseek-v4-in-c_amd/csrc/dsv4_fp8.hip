@@ -245,12 +245,12 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
          * the first weights' latency, so nothing here may wait for those: the
          * scales stay raw, no branch stands between the loads and the waits
          * that count them (lanes past x's end load and store its last
-         * piece), and the rounds are the row's own (XL 1: a row of at most 64
-         * threads, XL 2: any). With the scales decoded where loaded and four
-         * times the rounds, x was stored only once the weights had arrived
+         * piece), and the rounds are the row's own (XL: the row's waves, 1,
+         * 2 or 4). With the scales decoded where loaded and four times the
+         * rounds, x was stored only once the weights had arrived
          * (24576x1536 9.26 us, now 8.54). */
         float *xs = part + (size_t)(tc > 64 ? tc / 64 : 0) * rows_per_wg;
-        constexpr int XR = XL == 1 ? NCH : 4 * NCH;    /* rounds: cols <= 1024 XR */
+        constexpr int XR = XL ? XL * NCH : 1;          /* rounds: cols <= 1024 XR */
         f32x4 xv[XR], nv[NQ ? XR : 1];
         const int nq = cols >> 2;
         /* (NQ: the norm's weights with x, ahead of the weights' requests, and
@@ -314,6 +314,9 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
         load_step<NCH, R, SF>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb, sc, blk_r);
     }
 
+    uint32_t sv0[NCH];
+#pragma unroll
+    for (int n = 0; n < NCH; n++) sv0[n] = sv[n];
     for (int step = 0; step < nsteps; ++step) {
         const int rbase = row0 + step * step_rows + g * R;
         if (PF && step + 1 < nsteps)
@@ -359,6 +362,15 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
             load_step<NCH, R, SF>(wv, sv, W, S, rbase + step_rows, rend, cols, ch, j, tc, cb,
                                   sc, blk_r);
         }
+    }
+
+    /* A second use of the first step's raw scales, in no instruction. Without
+     * it the compiler carries E8M0 scales into the loop as bytes and widens
+     * them before it, behind a wait for the first weights that x's reads
+     * from LDS then stand behind. */
+    if (SF == 0 && XL) {
+#pragma unroll
+        for (int n = 0; n < NCH; n++) asm volatile("" ::"v"(sv0[n]));
     }
 
     if (tc > 64) {
@@ -525,15 +537,20 @@ struct Fp8Plan {
     size_t lds = 0;
 };
 
-Fp8Plan fp8_plan(const Fp8Geom &g, int R, int rows, int cols, int wgs_per_cu, int ngroups)
+Fp8Plan fp8_plan(const Fp8Geom &g, int R, int rows, int cols, int wgs_per_cu, int ngroups,
+                 bool lds_x = true)
 {
     Fp8Plan p;
-    /* x through LDS (one fetch per workgroup instead of one per row group)
-     * measured faster on MI355X for narrow rows (24576x1536: 12.2 -> 11.8
-     * us) and the widest (7168x16384: 24.8 -> 24.1 us), and within noise
-     * or slower between them. */
-    p.xl = g.wg == 256 && (cols & 3) == 0 &&
-           env_int("DSV4_GPU_FP8_XL", cols <= 2048 || cols >= 16384) != 0;
+    /* x through LDS: one fetch per workgroup instead of one per row group,
+     * and none of it waits for the first weights. Faster on every shape (us,
+     * each thread its own x from L2 / through LDS, fp32 scales and E8M0):
+     * 4096x4096 6.14 / 5.65 and 6.14 / 5.61, 512x4096 3.73 / 3.28 and 3.78 /
+     * 3.43, 32768x4096 25.0 / 23.6 and 25.1 / 23.7, 24576x2560 14.2 / 12.5
+     * and 14.2 / 12.7, 4096x8192 9.62 / 9.18 and 9.36 / 8.98, 7168x7168
+     * 11.87 / 11.63 and 12.15 / 12.02, 576x7168 4.36 / 4.21 and 4.39 / 4.27,
+     * 129280x7168 140.0 / 139.5 and 142.5 / 140.6. Rows of 192 threads,
+     * whose workgroup is not 256, read it from L2. */
+    p.xl = lds_x && g.wg == 256 && (cols & 3) == 0 && env_int("DSV4_GPU_FP8_XL", 1) != 0;
     const int step_rows = g.rg * R;
     const int nsteps = (rows + step_rows - 1) / step_rows;
     const int want = (wgs_per_cu * cu_count() + ngroups - 1) / ngroups;
@@ -564,10 +581,15 @@ void launch_gemv(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
                                  dsv4_lds_limit(), "fp8 gemv");
             (void)dsv4_lds_optin((const void *)k_fp8_gemv<NCH, R, SF, PF, 2>,
                                  dsv4_lds_limit(), "fp8 gemv");
+            (void)dsv4_lds_optin((const void *)k_fp8_gemv<NCH, R, SF, PF, 4>,
+                                 dsv4_lds_limit(), "fp8 gemv");
             opted = true;
         }
     }
-    if (xl && g.tc > 64)
+    if (xl && g.tc > 128)
+        hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 4>), dim3(grid, gp.n), dim3(g.wg), lds,
+                           st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
+    else if (xl && g.tc > 64)
         hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 2>), dim3(grid, gp.n), dim3(g.wg), lds,
                            st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
     else if (xl)
@@ -1218,15 +1240,18 @@ int dsv4_xproj_launch(const float *x, int cols, int sfmt, int blk_r, int blk_c, 
     }
     if (!ok) return two();
     const Fp8Valu v = fp8_valu(rmf, cols, blk_r, sfmt, false);
-    const Fp8Plan pf = fp8_plan(g, v.R, rmf, cols, v.wpc, nf);
+    const Fp8Plan pf = fp8_plan(g, v.R, rmf, cols, v.wpc, nf, false);
     /* the BF16 part within the FP8 part's grid (DSV4_GPU_XPROJ_CAP=0: its own
      * plan): a wider x grid only adds workgroups of one step each */
     const B16Plan pb = b16_plan(gb, rmb, nb, env_int("DSV4_GPU_XPROJ_CAP", 1) ? pf.grid : 0);
     /* the one combination built: FP8 with 4 chunks per thread, 2 rows per
-     * step, prefetch, x in registers; BF16 with 8 chunks per thread, 1 row
-     * (hidden 4096 and 7168, the Flash and full shapes) */
-    if (g.nch < 4 || v.R != 2 || !v.pf || pf.xl || gb.nch <= 4 || pb.R != 1 || g.wg != 256 ||
-        gb.wg != 256)
+     * step, prefetch, x in registers (through LDS the step measured slower:
+     * ratio 128 at 2200 positions 48.9 / 49.5 us, ratio 4 71.9 / 72.0; the
+     * second step's weights are then requested only after the first's
+     * arrive); BF16 with 8 chunks per thread, 1 row (hidden 4096 and 7168,
+     * the Flash and full shapes) */
+    if (g.nch < 4 || v.R != 2 || !v.pf || cols >= 16384 || gb.nch <= 4 || pb.R != 1 ||
+        g.wg != 256 || gb.wg != 256)
         return two();
     XProj a;
     a.x = x;
@@ -1294,7 +1319,7 @@ int dsv4_qproj_launch(const float *qr, int cols, const float *nw, float eps, int
      * the more of them there are the more weights are in flight meanwhile
      * (the CSA step above 75.6 -> 73.8 us). */
     const Fp8Plan pf = fp8_plan(g, qrr, rm, cols, v.wpc, 1);
-    /* the combinations built: x through LDS (cols <= 2048), 1 or 2 chunks
+    /* the combinations built: x through LDS, 1 or 2 chunks
      * per thread, 2 or 4 rows per step, no prefetch (wq_b's rows), 256
      * threads */
     if (!pf.xl || g.wg != 256 || g.nch > 2 || v.R != 2 || v.pf) return two();

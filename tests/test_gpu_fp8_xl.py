@@ -19,7 +19,8 @@ _KEEP = []          # resident matrices are keyed by host address
 @pytest.mark.parametrize("scales", ["e8m0", "f32"])
 @pytest.mark.parametrize("rows,cols", [
     (1, 16), (5, 48), (700, 512), (130, 1008), (64, 1024), (67, 1040), (1025, 1536),
-    (259, 2032), (2100, 2048), (33, 2064), (70, 4096), (37, 8192), (35, 16368), (300, 16384)])
+    (259, 2032), (2100, 2048), (33, 2064), (70, 4096), (66, 4112), (1300, 7168), (37, 8192),
+    (41, 12304), (35, 16368), (300, 16384)])
 def test_x_through_lds(gpu, dsv4, monkeypatch, rows, cols, scales):
     rng = np.random.default_rng(rows * 31 + cols)
     W = common.fp8_codes(rng, (rows, cols))
