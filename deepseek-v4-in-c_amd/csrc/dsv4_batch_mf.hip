@@ -51,6 +51,8 @@
 
 namespace {
 
+#include "dsv4_batch_walk.h"
+
 enum { MF_E8M0 = 0, MF_F32S = 1, MF_BF16 = 2, MF_FP4 = 3 };
 
 struct MfArgs {
@@ -197,11 +199,8 @@ k_batch_mf(const MfArgs a)
                    FULL ? c * CE * 4 : 0);
     };
 
-    /* a wave's steps: the groups of chunks j0 + 4 u + n tc inside the row, n
-     * fastest */
-    const int U = a.L >> 2, live_u = j0 < ch ? min(U, (ch - j0 + 3) >> 2) : 0;
-    int steps = 0;
-    for (int u = 0; u < live_u; u++) steps += nch - (j0 + 4 * u + (nch - 1) * tc < ch ? 0 : 1);
+    /* a wave's steps (dsv4_batch_walk.h) */
+    const int U = a.L >> 2, steps = mf_steps(j0, a.L, tc, ch, nch);
 
     /* (the chunk and ring slot of the next copy, of the next step) */
     int cu = 0, cc = j0, cs = 0, ci = 0;
@@ -309,11 +308,12 @@ k_batch_mf(const MfArgs a)
         u32x4 w, s4[2];
         f32x4 x[4][NX];
     } fe, fo;
-    int ru = 0, rn = 0, rc = j0, rs = 0, ri = 0;           /* the next step to read */
+    MfWalk rd(j0);                                         /* the next step to read */
+    int rs = 0, ri = 0;
     auto fetch = [&](Ops &f) {
         /* its copies have arrived; those of the steps after it may be in
-         * flight (past the last step: a read of nothing new, so that every
-         * pass makes the same reads and the waits count them) */
+         * flight (past the last step: a read of what lies there, so that
+         * every pass makes the same reads and the waits count them) */
         if (steps - 1 - ri >= 1) vm_wait<DPW>();
         else vm_wait<0>();
         const unsigned char *st = ring + rs * SB;
@@ -332,18 +332,13 @@ k_batch_mf(const MfArgs a)
             }
         }
         if (FMT == MF_FP4) {
-            f.s4[0] = *reinterpret_cast<const u32x4 *>(sl4 + (ru * nch + rn) * 128 + g * 32);
-            f.s4[1] = *reinterpret_cast<const u32x4 *>(sl4 + (ru * nch + rn) * 128 + g * 32 + 16);
+            const unsigned char *const s4 = sl4 + rd.entry(nch, groups) * 128 + g * 32;
+            f.s4[0] = *reinterpret_cast<const u32x4 *>(s4);
+            f.s4[1] = *reinterpret_cast<const u32x4 *>(s4 + 16);
         }
         rs = rs + 1 == DP ? 0 : rs + 1;
         ri++;
-        rn++;
-        rc += tc;
-        if (rc >= ch) {
-            ru++;
-            rn = 0;
-            rc = j0 + 4 * ru;
-        }
+        rd.next(j0, tc, ch);
     };
 
     int u = 0, n = 0, c0 = j0;
