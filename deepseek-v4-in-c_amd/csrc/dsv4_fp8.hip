@@ -834,15 +834,6 @@ int mf_split(const Fp8Geom &g, int rows, int nt)
     return tiles * 4 <= cu_count() ? 4 : tiles * 2 <= cu_count() ? 2 : 1;
 }
 
-/* the split tiles' block sums */
-size_t mf_scratch_bytes(int rows, int cols, int nt)
-{
-    Fp8Geom g;
-    if (rows <= 0 || nt < 2 || !fp8_geom(cols, &g)) return 0;
-    const int z = mf_split(g, rows, nt);
-    return z == 1 ? 0 : sizeof(float) * (size_t)std::max(z, g.tc / 64) * nt * rows;
-}
-
 template <int SF>
 void launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
                    const void *S, int rows, int cols, int sc, int blk_r,
@@ -1168,9 +1159,24 @@ int dsv4_fp8_gemv_groups_launch(float *y, const float *x, const uint8_t *W,
     return fp8_gemv(y, x, W, S, sfmt, rows, cols, blk_r, blk_c, gp, st);
 }
 
+bool dsv4_fp8_mx_form(int sfmt, int cols, int blk_r, int blk_c)
+{
+    return mx_form(sfmt, cols, blk_r, blk_c);
+}
+
+/* The split tiles' block sums. A split leaves at most one workgroup per CU
+ * (mf_split): on 256 CUs at most 128 tiles of 256 results, 4 sums of each. */
+size_t dsv4_fp8_n_split_bytes(int rows, int cols, int nt)
+{
+    Fp8Geom g;
+    if (rows <= 0 || nt < 2 || !fp8_geom(cols, &g)) return 0;
+    const int z = mf_split(g, rows, nt);
+    return z == 1 ? 0 : sizeof(float) * (size_t)std::max(z, g.tc / 64) * nt * rows;
+}
+
 size_t dsv4_fp8_n_scratch_bytes(int rows, int cols, int nt)
 {
-    return std::max(dsv4_fp8_mxn_scratch_bytes(cols, nt), mf_scratch_bytes(rows, cols, nt));
+    return std::max(dsv4_fp8_mxn_scratch_bytes(cols, nt), dsv4_fp8_n_split_bytes(rows, cols, nt));
 }
 
 int dsv4_fp8_gemv_n_launch(float *y, const float *x, const uint8_t *W,

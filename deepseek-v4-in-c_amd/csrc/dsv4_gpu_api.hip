@@ -25,6 +25,7 @@
 
 #include <algorithm>
 #include <map>
+#include <mutex>
 #include <vector>
 
 /* Scratch of dsv4_gpu_moe_fp4_noalloc_d: a fixed array in every device's
@@ -155,6 +156,43 @@ int scratch_reserve(Scratch &s, size_t bytes)
     HIP_OK(hipMemset(s.p, 0, bytes), "hipMemset scratch");
     s.cap = bytes;
     return 0;
+}
+
+/* The block sums of dsv4_gpu_fp8_gemv_n_d's split form (dsv4_fp8.hip), a slot
+ * per stream: calls on one stream follow each other, so a slot's next call
+ * comes after its last join, and calls on different streams never meet in one.
+ * A few streams' slots, allocated by dsv4_gpu_init and never moved or handed on
+ * until dsv4_gpu_shutdown. A call without a slot takes the unsplit form, which
+ * needs none and gives the same bits (1536x7168 at 13 tokens 15.4 us for 13.0):
+ * on a stream that comes after SPLIT_SLOTS others, and on hipStreamPerThread,
+ * one name for several streams. So does a call under capture, whose graph may
+ * be replayed on any stream, beside calls on the one it was captured on. */
+constexpr int SPLIT_SLOTS = 8;
+struct SplitPool {
+    std::mutex mu;
+    char *mem = nullptr;
+    int n = 0;                                   /* slots taken */
+    hipStream_t owner[SPLIT_SLOTS] = {};
+} g_split;
+
+void *split_slot(hipStream_t st, size_t bytes)
+{
+    if (!bytes || bytes > DSV4_FP8_SPLIT_MAX || st == hipStreamPerThread) return nullptr;
+    if (st) {                                    /* the default stream is never captured */
+        hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+        if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+            (void)hipGetLastError();
+            return nullptr;
+        }
+        if (cs != hipStreamCaptureStatusNone) return nullptr;
+    }
+    std::lock_guard<std::mutex> lock(g_split.mu);
+    if (!g_split.mem) return nullptr;
+    int i = 0;
+    while (i < g_split.n && g_split.owner[i] != st) i++;
+    if (i == SPLIT_SLOTS) return nullptr;
+    if (i == g_split.n) g_split.owner[g_split.n++] = st;
+    return g_split.mem + (size_t)i * DSV4_FP8_SPLIT_MAX;
 }
 
 /* A staged host-buffer call: inputs are packed into the pinned arena and
@@ -548,6 +586,9 @@ int dsv4_gpu_init(void)
         HIP_OK(hipGetSymbolAddress(&ptr, HIP_SYMBOL(moe_sync)), "hipGetSymbolAddress moe_sync");
         g_moe_sync[dev] = ptr;
     }
+    if (!g_split.mem)
+        HIP_OK(hipMalloc((void **)&g_split.mem, SPLIT_SLOTS * DSV4_FP8_SPLIT_MAX),
+               "hipMalloc split sums");
     printf("hip: %s (%s), %d CUs, %.2f GB free of %.2f GB\n", p.name,
            p.gcnArchName, p.multiProcessorCount, (double)freeb / 1073741824.0,
            (double)totb / 1073741824.0);
@@ -583,6 +624,9 @@ void dsv4_gpu_shutdown(void)
         s->p = nullptr;
         s->cap = 0;
     }
+    if (g_split.mem) (void)hipFree(g_split.mem);
+    g_split.mem = nullptr;
+    g_split.n = 0;
     if (g_ar.h) (void)hipHostFree(g_ar.h);
     if (g_ar.d) (void)hipFree(g_ar.d);
     g_ar = Arena{};
@@ -683,9 +727,16 @@ int dsv4_gpu_fp8_gemv_n_d(float *d_y, const float *d_x, const uint8_t *d_w,
         DSV4_ERR("fp8_gemv_n_d: bad arguments (nt %d)", nt);
         return -1;
     }
-    if (scratch_reserve(g_xsplit, dsv4_fp8_n_scratch_bytes(rows, cols, nt)) != 0) return -1;
-    return dsv4_fp8_gemv_n_launch(d_y, d_x, d_w, d_s, scale_fmt, rows, cols, 128, 128, nt,
-                                  as_stream(stream), g_xsplit.p);
+    hipStream_t st = as_stream(stream);
+    void *scr;
+    if (dsv4_fp8_mx_form(scale_fmt, cols, 128, 128)) {
+        if (scratch_reserve(g_xsplit, dsv4_fp8_mxn_scratch_bytes(cols, nt)) != 0) return -1;
+        scr = g_xsplit.p;
+    } else {
+        scr = split_slot(st, dsv4_fp8_n_split_bytes(rows, cols, nt));
+    }
+    return dsv4_fp8_gemv_n_launch(d_y, d_x, d_w, d_s, scale_fmt, rows, cols, 128, 128, nt, st,
+                                  scr);
 }
 
 int dsv4_gpu_fp4_gemv_d(float *d_y, const float *d_x, const uint8_t *d_w,

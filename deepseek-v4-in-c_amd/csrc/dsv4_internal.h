@@ -156,10 +156,14 @@ int dsv4_embed_row_launch(float *d_dst, const void *d_table, int wdt, long long 
                           int hidden, hipStream_t st);
 
 /* Batched: y[nt][rows], x[nt][cols]; per (row, token) bit-identical to the
- * GEMV above. xscratch: device memory of dsv4_fp8_n_scratch_bytes(rows, cols,
- * nt) bytes, for the E8M0 matrix-core form's split of x or the f32
- * matrix-core form's part sums (without it those forms fall back to kernels
- * that need none, with the same bits). */
+ * GEMV above. xscratch: device memory, dsv4_fp8_mxn_scratch_bytes for the
+ * E8M0 matrix-core form's split of x (_mx_form: the calls that run it) or
+ * _n_split_bytes (at most DSV4_FP8_SPLIT_MAX, 0 where tiles are not split) for
+ * the f32 matrix-core form's part sums; _n_scratch_bytes holds either. Without
+ * it those forms fall back to kernels that need none, with the same bits. */
+bool dsv4_fp8_mx_form(int sfmt, int cols, int blk_r, int blk_c);
+constexpr size_t DSV4_FP8_SPLIT_MAX = 512 * 1024;
+size_t dsv4_fp8_n_split_bytes(int rows, int cols, int nt);
 size_t dsv4_fp8_n_scratch_bytes(int rows, int cols, int nt);
 int dsv4_fp8_gemv_n_launch(float *y, const float *x, const uint8_t *W,
                            const void *S, int sfmt, int rows, int cols,

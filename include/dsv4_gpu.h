@@ -26,7 +26,7 @@
  *     weight pointer, which must stay stable (dsv4_cuda.cu:232-236).
  *   - Single-threaded: call from one host thread (the reference contract,
  *     dsv4_cuda.cu:243-249). Calls that overlap on one device race on the
- *     backend's staging and scratch buffers.
+ *     backend's staging and scratch buffers, but where a call says otherwise.
  *
  * Built with hipcc for gfx950 as libdsv4_gpu.so; a CPU-only build links
  * dsv4_gpu_stub.c instead, which defines every symbol below and reports no
@@ -140,8 +140,11 @@ int dsv4_gpu_fp8_gemv_d(float *d_y, const float *d_x, const uint8_t *d_w,
 /* The batched form (prefill, the k_mmq_fp8_n contract of dsv4_cuda.cu:161-
  * 230): d_y[nt][rows] for d_x[nt][cols], each (row, token) bit-identical to
  * dsv4_gpu_fp8_gemv_d on that token. nt <= DSV4_MAX_BATCH. What
- * dsv4_gpu_mmq_n runs after staging. The same alignment rule; its scratch
- * (x's term planes or part sums) is the library's, grown on demand. */
+ * dsv4_gpu_mmq_n runs after staging. The same alignment rule. Calls on
+ * different streams may overlap on the device (its part sums have a place per
+ * stream; a stream is idle when it is destroyed), and a captured call holds no
+ * library scratch. With DSV4_GPU_FP8_MX=1 neither is so: x's term planes are
+ * one library buffer, grown on demand. */
 int dsv4_gpu_fp8_gemv_n_d(float *d_y, const float *d_x, const uint8_t *d_w,
                           const void *d_s, int scale_fmt, int rows, int cols, int nt,
                           void *stream);
