@@ -834,10 +834,12 @@ int mf_split(const Fp8Geom &g, int rows, int nt)
     return tiles * 4 <= cu_count() ? 4 : tiles * 2 <= cu_count() ? 2 : 1;
 }
 
+/* 0; -1 where the f32 matrix-core form's launch failed, whose error it has
+ * taken (a failed launch of the others is still there for the caller to get) */
 template <int SF>
-void launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
-                   const void *S, int rows, int cols, int sc, int blk_r,
-                   int blk_c, int nt, hipStream_t st, void *scratch)
+int launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
+                  const void *S, int rows, int cols, int sc, int blk_r,
+                  int blk_c, int nt, hipStream_t st, void *scratch)
 {
     if (mf_takes(g, blk_r, nt)) {
         Dsv4BatchMf b;
@@ -847,7 +849,8 @@ void launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
         b.slots = mf_slots();
         b.split = mf_split(g, rows, nt);
         b.part = (float *)scratch;
-        if (dsv4_batch_mf_launch(b, st) <= 0) return;
+        const int rc = dsv4_batch_mf_launch(b, st);
+        if (rc <= 0) return rc;
     }
     /* two or more tokens: x through LDS, the largest token block that fits
      * and the tokens fill (8 x 4096, 4 x 7168, 2 x 16384 columns); three
@@ -856,9 +859,9 @@ void launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
     const size_t cap = dsv4_lds_limit() - 2048;
     if (nt >= 2 && (((uintptr_t)x) & 15) == 0 && g.tc <= 256 && 512 % g.tc == 0) {
         const size_t row4 = sizeof(float) * (size_t)cols;
-        if (nt >= 8 && 8 * row4 <= cap) { launch_gemv_nl_nch<SF, 8>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st); return; }
-        if (nt >= 3 && 4 * row4 <= cap) { launch_gemv_nl_nch<SF, 4>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st); return; }
-        if (2 * row4 <= cap) { launch_gemv_nl_nch<SF, 2>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st); return; }
+        if (nt >= 8 && 8 * row4 <= cap) { launch_gemv_nl_nch<SF, 8>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st); return 0; }
+        if (nt >= 3 && 4 * row4 <= cap) { launch_gemv_nl_nch<SF, 4>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st); return 0; }
+        if (2 * row4 <= cap) { launch_gemv_nl_nch<SF, 2>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st); return 0; }
     }
     const int grid = (rows + g.rg - 1) / g.rg;
     switch (g.nch) {
@@ -867,6 +870,7 @@ void launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
     case 3: hipLaunchKernelGGL((k_fp8_gemv_n<3, SF>), dim3(grid), dim3(g.wg), 0, st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, nt); break;
     default: hipLaunchKernelGGL((k_fp8_gemv_n<4, SF>), dim3(grid), dim3(g.wg), 0, st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, nt); break;
     }
+    return 0;
 }
 
 bool blocking_ok(int blk_r, int blk_c)
@@ -1198,10 +1202,11 @@ int dsv4_fp8_gemv_n_launch(float *y, const float *x, const uint8_t *W,
     Fp8Geom g;
     if (fp8_geom(cols, &g) && blocking_ok(blk_r, blk_c)) {
         if (chunked_ok(x, W, "fp8 gemv_n") != 0) return -1;
-        if (sfmt == 0)
-            launch_gemv_n<0>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st, xscratch);
-        else
-            launch_gemv_n<1>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st, xscratch);
+        if ((sfmt == 0 ? launch_gemv_n<0>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st,
+                                          xscratch)
+                       : launch_gemv_n<1>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st,
+                                          xscratch)) != 0)
+            return -1;
     } else {
         const int grid = (rows + 3) / 4;
         if (sfmt == 0)
