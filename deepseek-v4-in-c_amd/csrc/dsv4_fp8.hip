@@ -158,7 +158,7 @@ struct Fp8Groups {
  * unconditionally -- rows past the end read the last row, inactive chunks
  * the last chunk, and their results are discarded -- so no branch stands
  * between the loads and the waits that count them. */
-template <int NCH, int R, int SF>
+template <int NCH, int R, int SF, bool RAW>
 __device__ __forceinline__ void load_step(u32x4 (*wv)[NCH], uint32_t *sv, const uint8_t *W,
                                           const void *S, int rbase, int rend, int cols,
                                           int ch, int j, int tc, const int *cb, int sc,
@@ -175,8 +175,32 @@ __device__ __forceinline__ void load_step(u32x4 (*wv)[NCH], uint32_t *sv, const 
     }
     const int rb = min(rbase, rend - 1) / blk_r;
 #pragma unroll
-    for (int n = 0; n < NCH; n++) sv[n] = ld_scale_raw<SF>(S, (size_t)rb * sc + cb[n]);
+    for (int n = 0; n < NCH; n++) {
+        const uint32_t raw = ld_scale_raw<SF>(S, (size_t)rb * sc + cb[n]);
+        sv[n] = RAW ? raw : __float_as_uint(scale_val<SF>(raw));
+    }
 }
+
+/* Whether a step's scales stay as loaded until they are used (RAW) or are
+ * decoded where they are loaded; and whether the first step's loads stand
+ * behind a branch (HELD; always taken, a workgroup has rows) that keeps the
+ * compiler from mixing them with x's. Neither changes a result. A kernel
+ * whose x goes through LDS wants its scales raw and the loads free, so that
+ * x does not wait for the first weights; but each form was measured, cold, us:
+ *   - E8M0, x from L2: decoded and held (7168x12288 17.67 -> 17.09, 7168x7168
+ *     12.12 -> 11.69), but raw for three chunks and one row per step without
+ *     prefetch (4096x9216 12.71 -> 11.08, 5120x4608 8.91 -> 7.92);
+ *   - fp32, x from L2: held for one row per step (7168x7168 11.84 -> 11.50),
+ *     not for more (16384x12288 35.7 -> 34.2, 1536x12288 8.11 -> 7.90);
+ *   - rows of 256 threads through LDS: E8M0 decoded without prefetch
+ *     (7168x16384 21.65 -> 20.95), raw with it (4096x16384 14.21 -> 14.05);
+ *     fp32 held with prefetch (7168x16384 21.42 -> 20.77, 4096x16384 14.6 ->
+ *     14.1), free in one step (256x16384 4.74 -> 4.19). */
+template <int NCH, int R, int SF, int PF, int XL>
+struct Fp8Form {
+    static constexpr bool RAW = XL == 0 ? NCH == 3 && R == 1 && !PF : XL != 4 || PF;
+    static constexpr bool HELD = XL == 0 ? SF == 0 || R == 1 : XL == 4 && SF == 1 && PF;
+};
 
 /* One workgroup owns the contiguous rows [row0, row0 + rows_per_wg). It walks
  * them in steps of rg*R rows (row group g takes rows g*R .. g*R+R-1 of the
@@ -210,6 +234,8 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
         S = (const uint8_t *)S + gi * gp.s;
     }
 
+    constexpr bool RAW = Fp8Form<NCH, R, SF, PF, XL>::RAW;
+    constexpr bool HELD = Fp8Form<NCH, R, SF, PF, XL>::HELD;
     const int tid = threadIdx.x;
     const int g = tid / tc;
     const int j = tid - g * tc;
@@ -242,12 +268,12 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
          * would fetch the same x from L2.
          *
          * What is meant to overlap is x's way through LDS (and the norm) with
-         * the first weights' latency, so nothing here may wait for those: the
-         * scales stay raw, no branch stands between the loads and the waits
-         * that count them (lanes past x's end load and store its last
-         * piece), and the rounds are the row's own (XL: the row's waves, 1,
-         * 2 or 4). With the scales decoded where loaded and four times the
-         * rounds, x was stored only once the weights had arrived
+         * the first weights' latency, so nothing here should wait for those:
+         * the scales stay raw (Fp8Form), no branch stands between the loads
+         * and the waits that count them (lanes past x's end load and store
+         * its last piece), and the rounds are the row's own (XL: the row's
+         * waves, 1, 2 or 4). With the scales decoded where loaded and four
+         * times the rounds, x was stored only once the weights had arrived
          * (24576x1536 9.26 us, now 8.54). */
         float *xs = part + (size_t)(tc > 64 ? tc / 64 : 0) * rows_per_wg;
         constexpr int XR = XL ? XL * NCH : 1;          /* rounds: cols <= 1024 XR */
@@ -263,7 +289,9 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
             if (NQ) nv[q] = ldf4(nq_w + i);
         }
         __builtin_amdgcn_sched_barrier(0);
-        load_step<NCH, R, SF>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb, sc, blk_r);
+        if (!HELD || nsteps > 0)
+            load_step<NCH, R, SF, RAW>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb,
+                                       sc, blk_r);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int q = 0; q < XR; q++) {
@@ -311,7 +339,9 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
                 xr[n][q * 4 + 2] = v.z; xr[n][q * 4 + 3] = v.w;
             }
         }
-        load_step<NCH, R, SF>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb, sc, blk_r);
+        if (!HELD || nsteps > 0)
+            load_step<NCH, R, SF, RAW>(wv, sv, W, S, row0 + g * R, rend, cols, ch, j, tc, cb,
+                                       sc, blk_r);
     }
 
     uint32_t sv0[NCH];
@@ -320,8 +350,8 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
     for (int step = 0; step < nsteps; ++step) {
         const int rbase = row0 + step * step_rows + g * R;
         if (PF && step + 1 < nsteps)
-            load_step<NCH, R, SF>(wn, sn, W, S, rbase + step_rows, rend, cols, ch, j, tc, cb,
-                                  sc, blk_r);
+            load_step<NCH, R, SF, RAW>(wn, sn, W, S, rbase + step_rows, rend, cols, ch, j, tc,
+                                       cb, sc, blk_r);
 
         float acc[R];
 #pragma unroll
@@ -329,7 +359,8 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
             float a = 0.0f;
 #pragma unroll
             for (int n = 0; n < NCH; n++) {
-                const float d = fmaf(dot16(wv[i][n], xr[n]), scale_val<SF>(sv[n]), a);
+                const float sf = RAW ? scale_val<SF>(sv[n]) : __uint_as_float(sv[n]);
+                const float d = fmaf(dot16(wv[i][n], xr[n]), sf, a);
                 a = act[n] ? d : a;
             }
             acc[i] = a;
@@ -359,8 +390,8 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
 #pragma unroll
             for (int n = 0; n < NCH; n++) sv[n] = sn[n];
         } else if (step + 1 < nsteps) {
-            load_step<NCH, R, SF>(wv, sv, W, S, rbase + step_rows, rend, cols, ch, j, tc, cb,
-                                  sc, blk_r);
+            load_step<NCH, R, SF, RAW>(wv, sv, W, S, rbase + step_rows, rend, cols, ch, j, tc,
+                                       cb, sc, blk_r);
         }
     }
 
@@ -368,7 +399,7 @@ __device__ __forceinline__ void fp8_rows(float *__restrict__ y, const float *__r
      * it the compiler carries E8M0 scales into the loop as bytes and widens
      * them before it, behind a wait for the first weights that x's reads
      * from LDS then stand behind. */
-    if (SF == 0 && XL) {
+    if (SF == 0 && XL && RAW) {
 #pragma unroll
         for (int n = 0; n < NCH; n++) asm volatile("" ::"v"(sv0[n]));
     }
@@ -537,20 +568,41 @@ struct Fp8Plan {
     size_t lds = 0;
 };
 
-Fp8Plan fp8_plan(const Fp8Geom &g, int R, int rows, int cols, int wgs_per_cu, int ngroups,
-                 bool lds_x = true)
+/* Whether a row's x goes through LDS, one fetch per workgroup instead of one
+ * per row group (steps: a workgroup's). Rows of up to 64 threads: always (us,
+ * cold, each thread its own x from L2 / through LDS: 4096x4096 5.99 / 5.57,
+ * 512x4096 3.73 / 3.28, 32768x4096 25.0 / 23.6, 24576x1536 9.68 / 9.25). Wider
+ * rows have fewer row groups to share it, and each group's rounds of 1024
+ * columns cost their latency whether x fills them or not (full: it does):
+ *   - 128 threads, E8M0: where a step has four rows or the next one is
+ *     prefetched (1536x7168 5.71 / 5.56, 2560x4608 6.51 / 5.93), or four
+ *     chunks fill the rounds (2048x8192 6.63 / 6.30; 7168x7168 11.7 / 12.0,
+ *     8192x4608 9.44 / 9.85, 1024x4608 3.96 / 4.39);
+ *   - 128 threads, fp32: not for one row per step (512x4608 3.58 / 3.79,
+ *     5120x4608 7.70 / 8.18), but where four chunks fill the rounds (512x8192
+ *     3.95 / 3.77), and with prefetch where the rounds are full or there are
+ *     four chunks (4096x5120 6.92 / 7.19; 2048x7168 6.03 / 5.93);
+ *   - 256 threads: but for single steps whose rounds are not full (256x13312
+ *     fp32 4.05 / 4.39; 4096x13312 14.5 / 12.2, 1024x16384 7.4 / 6.8).
+ * Rows of 192 threads, whose workgroup is not 256, read it from L2. */
+bool fp8_xl(const Fp8Geom &g, int R, int pf, int sfmt, int cols, int steps)
+{
+    if (g.wg != 256 || (cols & 3)) return false;
+    const int waves = g.tc > 64 ? g.tc / 64 : 1;
+    const bool full = cols > 1024 * (waves * g.nch - 1);
+    bool xl = true;
+    if (waves == 2)
+        xl = R == 4 || (g.nch == 4 && full) ||
+             (sfmt == 0 ? pf != 0 : R == 2 && (!pf || full || g.nch == 4));
+    else if (waves == 4)
+        xl = full || steps > 1;
+    return env_int("DSV4_GPU_FP8_XL", xl) != 0;
+}
+
+Fp8Plan fp8_plan(const Fp8Geom &g, int R, int pf, int sfmt, int rows, int cols, int wgs_per_cu,
+                 int ngroups, bool lds_x = true)
 {
     Fp8Plan p;
-    /* x through LDS: one fetch per workgroup instead of one per row group,
-     * and none of it waits for the first weights. Faster on every shape (us,
-     * each thread its own x from L2 / through LDS, fp32 scales and E8M0):
-     * 4096x4096 6.14 / 5.65 and 6.14 / 5.61, 512x4096 3.73 / 3.28 and 3.78 /
-     * 3.43, 32768x4096 25.0 / 23.6 and 25.1 / 23.7, 24576x2560 14.2 / 12.5
-     * and 14.2 / 12.7, 4096x8192 9.62 / 9.18 and 9.36 / 8.98, 7168x7168
-     * 11.87 / 11.63 and 12.15 / 12.02, 576x7168 4.36 / 4.21 and 4.39 / 4.27,
-     * 129280x7168 140.0 / 139.5 and 142.5 / 140.6. Rows of 192 threads,
-     * whose workgroup is not 256, read it from L2. */
-    p.xl = lds_x && g.wg == 256 && (cols & 3) == 0 && env_int("DSV4_GPU_FP8_XL", 1) != 0;
     const int step_rows = g.rg * R;
     const int nsteps = (rows + step_rows - 1) / step_rows;
     const int want = (wgs_per_cu * cu_count() + ngroups - 1) / ngroups;
@@ -561,6 +613,7 @@ Fp8Plan fp8_plan(const Fp8Geom &g, int R, int rows, int cols, int wgs_per_cu, in
     if (spw < 1) spw = 1;
     p.rows_per_wg = spw * step_rows;
     p.grid = (rows + p.rows_per_wg - 1) / p.rows_per_wg;
+    p.xl = lds_x && fp8_xl(g, R, pf, sfmt, cols, spw);
     p.lds = (g.tc > 64 ? sizeof(float) * (size_t)wpr * p.rows_per_wg : 0)
           + (p.xl ? sizeof(float) * (size_t)cols : 0);
     return p;
@@ -571,7 +624,7 @@ void launch_gemv(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
                  const void *S, int rows, int cols, int sc, int blk_r,
                  int blk_c, int wgs_per_cu, const Fp8Groups &gp, hipStream_t st)
 {
-    const Fp8Plan p = fp8_plan(g, R, rows, cols, wgs_per_cu, gp.n);
+    const Fp8Plan p = fp8_plan(g, R, PF, SF, rows, cols, wgs_per_cu, gp.n);
     const int xl = p.xl, rows_per_wg = p.rows_per_wg, grid = p.grid;
     const size_t lds = p.lds;
     if (xl) {
@@ -918,7 +971,8 @@ int chunked_ok(const float *x, const uint8_t *W, const char *what)
  * prefetch on/off; x through LDS or not; 1-8 workgroups per CU; cold, us):
  *   - two workgroups per CU (four when rows are narrow, cols < 4096);
  *   - rows of 16384 columns with fp32 scales: one row per step with the
- *     next prefetched (7168x16384: 21.7-22.2 -> 21.1-21.3); with E8M0
+ *     next, if there is one, prefetched (7168x16384: 21.7-22.2 -> 21.1-21.3);
+ *     with E8M0
  *     scales the base below (21.2-21.4 against 22.4-22.5 for one row);
  *   - more than 4096 rows: two rows per step without prefetch, unless that
  *     grid leaves its last round of workgroups short, so that some CUs get
@@ -953,15 +1007,16 @@ Fp8Valu fp8_valu(int rows, int cols, int blk_r, int sfmt, bool tuned = true)
         const int cu = cu_count();
         /* every round of workgroups but the last is full; the last at least
          * 15/16 full, or the grid is a single round */
-        auto grid = [&](int r) { return fp8_plan(g, r, rows, cols, v.wpc, 1).grid; };
+        auto grid = [&](int r) { return fp8_plan(g, r, 0, sfmt, rows, cols, v.wpc, 1, false).grid; };
         auto full = [&](int r) {
             const int n = grid(r), last = n % cu;
             return n <= cu || last == 0 || last * 16 >= cu * 15;
         };
         if (g.tc == 256) {
             if (sfmt != 0) {
+                const Fp8Plan p = fp8_plan(g, 1, 0, sfmt, rows, cols, v.wpc, 1, false);
                 R = 1;
-                pf = 1;
+                pf = p.rows_per_wg > g.rg;
             }
         } else if (rows > 4096) {
             if (!full(2) && full(1)) R = 1;
@@ -1251,7 +1306,7 @@ int dsv4_xproj_launch(const float *x, int cols, int sfmt, int blk_r, int blk_c, 
     }
     if (!ok) return two();
     const Fp8Valu v = fp8_valu(rmf, cols, blk_r, sfmt, false);
-    const Fp8Plan pf = fp8_plan(g, v.R, rmf, cols, v.wpc, nf, false);
+    const Fp8Plan pf = fp8_plan(g, v.R, v.pf, sfmt, rmf, cols, v.wpc, nf, false);
     /* the BF16 part within the FP8 part's grid (DSV4_GPU_XPROJ_CAP=0: its own
      * plan): a wider x grid only adds workgroups of one step each */
     const B16Plan pb = b16_plan(gb, rmb, nb, env_int("DSV4_GPU_XPROJ_CAP", 1) ? pf.grid : 0);
@@ -1329,7 +1384,7 @@ int dsv4_qproj_launch(const float *qr, int cols, const float *nw, float eps, int
      * workgroup's norm stands between its first weights and the rest, and
      * the more of them there are the more weights are in flight meanwhile
      * (the CSA step above 75.6 -> 73.8 us). */
-    const Fp8Plan pf = fp8_plan(g, qrr, rm, cols, v.wpc, 1);
+    const Fp8Plan pf = fp8_plan(g, qrr, 0, sfmt, rm, cols, v.wpc, 1);
     /* the combinations built: x through LDS, 1 or 2 chunks
      * per thread, 2 or 4 rows per step, no prefetch (wq_b's rows), 256
      * threads */
