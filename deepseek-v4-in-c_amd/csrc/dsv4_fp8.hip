@@ -625,32 +625,22 @@ void launch_gemv(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
                  int blk_c, int wgs_per_cu, const Fp8Groups &gp, hipStream_t st)
 {
     const Fp8Plan p = fp8_plan(g, R, PF, SF, rows, cols, wgs_per_cu, gp.n);
-    const int xl = p.xl, rows_per_wg = p.rows_per_wg, grid = p.grid;
-    const size_t lds = p.lds;
-    if (xl) {
-        static bool opted = false;                  /* x of up to 64 KB + partials */
-        if (!opted) {
-            (void)dsv4_lds_optin((const void *)k_fp8_gemv<NCH, R, SF, PF, 1>,
-                                 dsv4_lds_limit(), "fp8 gemv");
-            (void)dsv4_lds_optin((const void *)k_fp8_gemv<NCH, R, SF, PF, 2>,
-                                 dsv4_lds_limit(), "fp8 gemv");
-            (void)dsv4_lds_optin((const void *)k_fp8_gemv<NCH, R, SF, PF, 4>,
-                                 dsv4_lds_limit(), "fp8 gemv");
-            opted = true;
+    auto go = [&](auto kern, bool *opted) {
+        if (opted && !*opted) {                     /* x of up to 64 KB + partials */
+            (void)dsv4_lds_optin((const void *)kern, dsv4_lds_limit(), "fp8 gemv");
+            *opted = true;
         }
-    }
-    if (xl && g.tc > 128)
-        hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 4>), dim3(grid, gp.n), dim3(g.wg), lds,
-                           st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
-    else if (xl && g.tc > 64)
-        hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 2>), dim3(grid, gp.n), dim3(g.wg), lds,
-                           st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
-    else if (xl)
-        hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 1>), dim3(grid, gp.n), dim3(g.wg), lds,
-                           st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
-    else
-        hipLaunchKernelGGL((k_fp8_gemv<NCH, R, SF, PF, 0>), dim3(grid, gp.n), dim3(g.wg), lds,
-                           st, y, x, W, S, rows, cols, sc, blk_r, blk_c, g.tc, rows_per_wg, gp);
+        hipLaunchKernelGGL(kern, dim3(p.grid, gp.n), dim3(g.wg), p.lds, st, y, x, W, S, rows,
+                           cols, sc, blk_r, blk_c, g.tc, p.rows_per_wg, gp);
+    };
+    static bool opted[3] = {};
+    if (!p.xl) return go(k_fp8_gemv<NCH, R, SF, PF, 0>, nullptr);
+    /* fp8_geom: two waves per row have 3 or 4 chunks per thread, four 4 */
+    if constexpr (NCH == 4)
+        if (g.tc > 128) return go(k_fp8_gemv<NCH, R, SF, PF, 4>, &opted[2]);
+    if constexpr (NCH >= 3)
+        if (g.tc > 64) return go(k_fp8_gemv<NCH, R, SF, PF, 2>, &opted[1]);
+    go(k_fp8_gemv<NCH, R, SF, PF, 1>, &opted[0]);
 }
 
 template <int R, int SF, int PF>
