@@ -511,22 +511,40 @@ int mf_fmt(MfArgs &a, bool sc1, bool full, hipStream_t st)
 }
 
 /* The waves a row tile's slots are split over. While every tile has a CU to
- * itself the most (16; 8 for FP4, whose two register sets take 256 VGPRs): a
- * tile's time is its own chain (us, P 16 / 8: FP8 2048x4096 at 16 tokens 11.1
- * / 11.4, BF16 1024x4096 at 48 10.9 / 12.2, 1024x7168 16.6 / 18.9). With more
- * tiles, fewer, so that several workgroups share a CU's LDS and one starts
- * while another ends (FP8 7168x7168 at 64 tokens P 16 / 8 / 4: 100.6 / 81.5 /
- * 84.2, 24576x1536 at 64 116.5 / 71.3 / 67.5; BF16 16384x4096 at 64 162.2 /
- * 123.9 / 117.4; FP4 P 8 / 4: 8192x8192 at 64 129.7 / 108.9). */
-int mf_waves(int fmt, int tc, long long tiles)
+ * itself the most (16; 8 for FP4, whose two register sets take 173 to 185
+ * VGPRs, too many for two such workgroups on a CU): a tile's time is its own
+ * chain (us, P 16 / 8: FP8 2048x4096 at 16 tokens 11.1 / 11.4, BF16 1024x4096
+ * at 48 10.9 / 12.2, 1024x7168 16.6 / 18.9). With more tiles, fewer, so that
+ * several workgroups share a CU's LDS and one starts while another ends (FP8
+ * 7168x7168 at 64 tokens P 16 / 8 / 4: 100.6 / 81.5 / 84.2, 24576x1536 at 64
+ * 116.5 / 71.3 / 67.5; BF16 16384x4096 at 64 162.2 / 123.9 / 117.4; FP4 P 8 /
+ * 4: 8192x8192 at 64 129.7 / 108.9).
+ * 192 slots divide into 12, 6 or 3 waves, of which 6 leave the LDS of half a
+ * CU unused: 12 up to three rounds of tiles, then 3 (us, P 12 / 6 / 3: 3072x
+ * 12288 at 48 tokens, 576 tiles, 70.7 / 79.5 / 84.3; 4096x12288 at 64, 1024
+ * tiles, 94.7 / 123.6 / 85.6); rows whose chunks do not end on a step (!full)
+ * keep 6 in the third round (12288x8208 at 16 59.6 / 57.4). Split over three
+ * workgroups (mf_split in dsv4_fp8.hip) with more tiles than CUs, 4 each
+ * (5120x12288 at 16 tokens P 16 / 8 / 4 / 2: 45.6 / 36.1 / 34.6 / 37.3). */
+int mf_waves(int fmt, int tc, bool full, bool split, long long tiles)
 {
     if (tiles <= 256) return fmt == MF_FP4 ? 8 : 16;
     if (fmt == MF_FP4) return 4;
     if (fmt == MF_BF16) return tiles <= 512 ? 8 : 4;
+    if (tc == 192) return split ? 4 : tiles <= (full ? 800 : 512) ? 12 : tiles <= 800 ? 8 : 3;
     return tc < 64 || (tc == 64 && tiles > 2048) ? 4 : 8;
 }
 
 } // namespace
+
+/* Rows of 192 slots: with the row tiles rounded up to the grid's eight per
+ * XCD, as one more than an XCD's CUs is a second round there (1360x12288 at 33
+ * tokens, 255 tiles: 45.6 us unsplit). */
+long long dsv4_batch_mf_tiles(int rows, int nt, int tc)
+{
+    const long long rt = ((long long)rows + 15) / 16;
+    return (tc == 192 ? (rt + 7) / 8 * 8 : rt) * ((nt + 15) / 16);
+}
 
 int dsv4_batch_mf_launch(const Dsv4BatchMf &b, hipStream_t st)
 {
@@ -544,10 +562,11 @@ int dsv4_batch_mf_launch(const Dsv4BatchMf &b, hipStream_t st)
     a.sc = b.sc; a.blk_r = b.blk_r; a.blk_c = b.blk_c;
     const bool f8 = b.fmt == MF_E8M0 || b.fmt == MF_F32S;
     if (f8 && (b.blk_r & 15)) return 1;
-    /* P waves per row tile (see MF_P): the smallest part of at least 4 slots,
+    /* P waves per row tile (mf_waves): the smallest part of at least 4 slots,
      * at most the 64 of one block of the tree */
-    const int want = mf_waves(b.fmt, a.tc, (long long)((b.rows + 15) / 16) * ((b.nt + 15) / 16));
     const int Z = b.split > 1 && b.part ? b.split : 1;
+    const bool full = a.ch % 4 == 0;
+    const int want = mf_waves(b.fmt, a.tc, full, Z > 1, dsv4_batch_mf_tiles(b.rows, b.nt, a.tc));
     int L = 4;
     while (a.tc / L / Z > want && 2 * L <= 64 && 2 * L <= a.tc) L *= 2;
     if (b.slots) L = b.slots;
@@ -562,7 +581,6 @@ int dsv4_batch_mf_launch(const Dsv4BatchMf &b, hipStream_t st)
     a.P = P; a.Z = Z;
     a.part = b.part;
     a.bc_m = b.blk_c > 0 ? (uint32_t)(((1ull << 32) + b.blk_c - 1) / b.blk_c) : 0;
-    const bool full = a.ch % 4 == 0;
     const bool sc1 = b.fmt == MF_BF16 ||
                      (f8 ? b.blk_c % 64 == 0
                          : full && b.blk_r == 1 && b.blk_c == 32 && (((uintptr_t)b.S) & 3) == 0);

@@ -848,33 +848,45 @@ void launch_gemv_nl_nch(const Fp8Geom &g, float *y, const float *x, const uint8_
  *
  * The batched GEMV's plan on the f32 matrix core (dsv4_batch_mf.hip, the
  * GEMV's bits): whether it runs, and the workgroups per tile of 16 rows x 16
- * tokens. It takes batches of 5 tokens on (8 where a row has 192 threads,
- * which k_fp8_gemv_nl does not take): below that its tile is mostly empty
+ * tokens. It takes batches of 5 tokens on: below that its tile is mostly empty
  * columns (us, matrix core / VALU, E8M0: 7168x7168 at 4 tokens 27.4 / 24.0, 6
  * tokens 28.0 / 43.6, 64 tokens 81.5 / 334.7; 1536x7168 at 4 tokens 12.9 /
- * 10.1, at 6 12.9 / 15.9; 512x12288 at 5 tokens 12.7 / 10.6, at 8 13.1 /
- * 14.9). While the tiles leave CUs idle, rows of 4096 columns on are split
+ * 10.1, at 6 12.9 / 15.9; of 1360 shapes of 16 to 24576 rows and 64 to 16384
+ * columns none of 5 tokens or more was slower than before). Rows of 192
+ * threads, which k_fp8_gemv_nl does not take: from 8 tokens, few of them from
+ * 9 or 11 (64x8208 at 8 tokens 10.5 / 8.2, at 10 10.6 / 10.1; 256x12288 at 9
+ * 12.9 / 12.0, at 12 12.9 / 14.6; 512x10240 at 8 13.2 / 12.9).
+ *
+ * While the tiles leave CUs idle, rows of 4096 columns on are split
  * over 4, 3 or 2 workgroups (a row's 64-slot blocks, or parts of one) that a
  * second launch joins: a tile's time is its chain down the row, and half of
  * it is worth more than the launch (us, split by 1 / 2 / 4: 1536x7168 at 13
  * tokens 15.4 / 13.4 / -, 576x7168 at 16 14.9 / 12.7 / 9.4, 1024x16384 at 16
  * 29.8 / 21.5 / 15.0, 2048x4096 at 16 11.0 / 10.1 / -; at 512x2048 no gain,
- * 7.1 / 7.1 / 7.1). DSV4_GPU_MFN_L (slots per wave) takes the form at any
+ * 7.1 / 7.1 / 7.1). Rows of 192 threads also while the tiles are a few more
+ * than the CUs, up to four thirds: thirds of a tile even out what whole tiles
+ * leave to a second round (5120x12288 at 16 tokens 48.8 / 34.6 by 3, 5120x
+ * 9216 38.4 / 28.1). DSV4_GPU_MFN_L (slots per wave) takes the form at any
  * batch, unsplit. */
 int mf_slots() { return env_int("DSV4_GPU_MFN_L", 0); }
 
-bool mf_takes(const Fp8Geom &g, int blk_r, int nt)
+bool mf_takes(const Fp8Geom &g, int rows, int blk_r, int nt)
 {
+    const int from = g.tc != 192 ? 5 : rows <= 256 ? 11 : rows <= 512 ? 9 : 8;
     return env_int("DSV4_GPU_FP8_MFN", 1) != 0 && nt >= 2 && g.tc >= 4 && (blk_r & 15) == 0 &&
-           (mf_slots() != 0 || nt >= (g.tc == 192 ? 8 : 5));
+           (mf_slots() != 0 || nt >= from);
 }
 
 int mf_split(const Fp8Geom &g, int rows, int nt)
 {
     const long long tiles = (long long)((rows + 15) / 16) * ((nt + 15) / 16);
+    const int cu = cu_count();
     if (mf_slots() != 0 || g.ch < 256 || g.tc < 64) return 1;
-    if (g.tc == 192) return tiles * 3 <= cu_count() ? 3 : 1;
-    return tiles * 4 <= cu_count() ? 4 : tiles * 2 <= cu_count() ? 2 : 1;
+    if (g.tc == 192) {
+        const long long t = dsv4_batch_mf_tiles(rows, nt, g.tc);
+        return tiles * 3 <= cu || (t > cu && t * 3 <= 4 * cu) ? 3 : 1;
+    }
+    return tiles * 4 <= cu ? 4 : tiles * 2 <= cu ? 2 : 1;
 }
 
 /* 0; -1 where the f32 matrix-core form's launch failed, whose error it has
@@ -884,7 +896,7 @@ int launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
                   const void *S, int rows, int cols, int sc, int blk_r,
                   int blk_c, int nt, hipStream_t st, void *scratch)
 {
-    if (mf_takes(g, blk_r, nt)) {
+    if (mf_takes(g, rows, blk_r, nt)) {
         Dsv4BatchMf b;
         b.fmt = SF; b.y = y; b.x = x; b.W = W; b.S = S;
         b.rows = rows; b.cols = cols; b.nt = nt;
@@ -1213,8 +1225,8 @@ bool dsv4_fp8_mx_form(int sfmt, int cols, int blk_r, int blk_c)
     return mx_form(sfmt, cols, blk_r, blk_c);
 }
 
-/* The split tiles' block sums. A split leaves at most one workgroup per CU
- * (mf_split): on 256 CUs at most 128 tiles of 256 results, 4 sums of each. */
+/* The split tiles' block sums (mf_split): on 256 CUs at most 128 tiles of 256
+ * results, 4 sums of each, or of rows of 192 threads 336 tiles, 3 of each. */
 size_t dsv4_fp8_n_split_bytes(int rows, int cols, int nt)
 {
     Fp8Geom g;

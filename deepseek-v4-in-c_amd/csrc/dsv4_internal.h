@@ -145,6 +145,8 @@ struct Dsv4BatchMf {
     float *part = nullptr;
 };
 int dsv4_batch_mf_launch(const Dsv4BatchMf &b, hipStream_t st);
+/* The tiles of 16 rows and 16 tokens that its plan goes by. */
+long long dsv4_batch_mf_tiles(int rows, int nt, int tc);
 
 /* Greedy argmax (the first index of the maximum, dsv4_run.c:471-472) over
  * d_v[n] into d_out[0]; scratch of dsv4_argmax_scratch_bytes. 0 / -1. */
@@ -162,7 +164,7 @@ int dsv4_embed_row_launch(float *d_dst, const void *d_table, int wdt, long long 
  * the f32 matrix-core form's part sums; _n_scratch_bytes holds either. Without
  * it those forms fall back to kernels that need none, with the same bits. */
 bool dsv4_fp8_mx_form(int sfmt, int cols, int blk_r, int blk_c);
-constexpr size_t DSV4_FP8_SPLIT_MAX = 512 * 1024;
+constexpr size_t DSV4_FP8_SPLIT_MAX = 1024 * 1024;
 size_t dsv4_fp8_n_split_bytes(int rows, int cols, int nt);
 size_t dsv4_fp8_n_scratch_bytes(int rows, int cols, int nt);
 int dsv4_fp8_gemv_n_launch(float *y, const float *x, const uint8_t *W,

@@ -19,14 +19,15 @@ def call(stream, rows, cols, nt, capture=0):
 streams = [None] + [names[i:].ctypes.data for i in range(12)]
 seen = {}
 for rep, (rows, cols, nt) in enumerate([(512, 4096, 16), (1024, 16384, 16), (1536, 7168, 13),
-                                        (300, 12288, 9), (2048, 16384, 16)]):
+                                        (300, 12288, 9), (2048, 16384, 16), (5376, 12288, 16)]):
     for i, s in enumerate(streams):
         p = call(s, rows, cols, nt)
         assert seen.setdefault(i, p) == p, ("moved", i, rep)
 own = sorted(p for p in seen.values() if p)
 assert len(set(own)) == len(own), own
-# 2048 x 16384 at 16 tokens: 128 tiles, the most that are split, four sums each
-assert all(b - a >= 4 * 16 * 2048 * 4 for a, b in zip(own, own[1:])), own
+# the most: 128 tiles of 2048 x 16384 with four sums each, 336 of 12288 columns with
+# three
+assert all(b - a >= 4 * max(4 * 16 * 2048, 3 * 16 * 5376) for a, b in zip(own, own[1:])), own
 assert shim.shim_frees() == 0
 for s in streams[1:]:
     assert call(s, 1536, 7168, 13, capture=1) is None and shim.shim_launches() == 1

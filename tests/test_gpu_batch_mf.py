@@ -56,6 +56,17 @@ def test_fp8(gpu, dsv4, rows, cols, nt, scales):
     _check(dsv4, m, _x(rng, nt, cols), ("fp8", rows, cols, nt, scales))
 
 
+# rows of 192 slots: split over 3 workgroups below and above one tile per CU
+# (4200 rows; 1360 at 33 tokens by the grid's eight row tiles per XCD), 12 waves
+# a tile, 6 (8208: a ragged last group), 3, and the least tokens of few rows
+@pytest.mark.parametrize("scales", ["e8m0", "f32"])
+@pytest.mark.parametrize("rows,cols,nt", [
+    (250, 9216, 11), (500, 10240, 9), (1360, 12288, 33), (4200, 8224, 16), (3000, 9216, 48),
+    (2200, 8208, 64), (4100, 9216, 64), (4100, 8208, 64)])
+def test_fp8_192_slots(gpu, dsv4, rows, cols, nt, scales):
+    test_fp8(gpu, dsv4, rows, cols, nt, scales)
+
+
 @pytest.mark.parametrize("blk_r,blk_c", [(16, 16), (16, 48), (32, 64), (128, 4096)])
 def test_fp8_blockings(gpu, dsv4, blk_r, blk_c):
     rows, cols, nt = 75, 2064, 18
