@@ -236,18 +236,46 @@ void f4n_launch(float *y, const float *x, const uint8_t *W, const uint8_t *S, in
 }
 
 /* From how many tokens the batch runs on the f32 matrix core
- * (dsv4_batch_mf.hip, the same bits): its time hardly depends on the tokens
- * of a tile of 16, k_fp4_gemv_n's grows with each (us, matrix core /
- * k_fp4_gemv_n: 7168x2048 at 3 tokens 10.6 / 9.1, at 4 10.5 / 11.0;
- * 2048x7168 at 3 15.3 / 15.3, at 4 15.4 / 19.1, at 24 16.4 / 102; 512x16384
- * at 4 29.4 / 27.5, at 5 29.5 / 34.0; 64x7168 at 4 14.7 / 12.6, at 5 14.8 /
- * 15.5; 64x2048 at 6 6.8 / 6.8; 8192x8192 at 2 32.8 / 44.8, at 64 109 /
- * 1242). */
-bool f4n_mf(int rows, int cols, int nt)
+ * (dsv4_batch_mf.hip, the same bits). Its time hardly depends on the tokens
+ * of a tile of 16, but steps up where the tiles of 16 rows pass one a CU, and
+ * two for every further round; k_fp4_gemv_n's is a few us plus so much per
+ * token, and grows with the rows from one workgroup a CU on (2048 rows; 1024
+ * above 4096 columns, where a workgroup has half as many). So the line lies
+ * high where the VALU has no second workgroup and where a round of tiles has
+ * only begun, low where a round is full (us, matrix core / k_fp4_gemv_n):
+ *   - above 2048 columns: 1024x7168 at 4 tokens 15.0 / 12.5, 2048x3584 at 4
+ *     11.1 / 9.9, 256x8192 at 5 17.7 / 17.3, 1024x4096 at 5 12.5 / 14.6;
+ *     2048x7168 at 4 15.6 / 18.8; 8192x8192 at 2 32.8 / 44.8;
+ *   - up to 2048 columns, one chunk per lane, where the tile's waves have a
+ *     step or two each: 2048x1536 at 4 7.7 / 5.1, at 9 7.9 / 8.3; 4096x512 at
+ *     4 5.8 / 4.7, at 7 5.8 / 6.2; 6144x1024 at 4 10.7 / 7.1, at 8 10.6 /
+ *     10.5; 8192x1024 at 6 10.7 / 10.3, at 7 10.7 / 11.3; 10240x512 at 9
+ *     13.6 / 13.1; 8192x2048 at 4 11.6 / 11.7.
+ * Of 4620 shapes of 16 to 16384 rows, 128 to 16384 columns and 2 to 12 tokens
+ * none is more than 5 % slower than on k_fp4_gemv_n. Where the tile reads its scales byte by byte (not 1x32 blocks, or a ragged last
+ * step) it starts a token later (64x8192 of 32x64 blocks at 5 tokens 18.4 /
+ * 17.2, 512x4128 at 5 12.5 / 11.8). */
+int f4n_from(int rows, int cols)
 {
-    if (cols <= 2048 && rows < 1024) return nt >= 7;
-    if (rows < 1024) return nt >= 5;
-    return nt >= (rows >= 8192 && cols >= 8192 ? 2 : 4);
+    const bool solo = rows <= (cols > 4096 ? 1024 : 2048);     /* a workgroup a CU */
+    if (cols > 2048) return solo ? 5 : rows >= 8192 && cols >= 8192 ? 2 : 4;
+    /* columns up to; one workgroup a CU, one tile a CU, the first round of
+     * two tiles a CU up to 3/4 full, any round fuller, a later one emptier */
+    static const struct { int cols, solo, one, two, full, more; } F[] = {
+        {128, 6, 5, 4, 4, 4},  {256, 9, 7, 6, 5, 7},  {512, 9, 7, 8, 7, 10},
+        {1024, 9, 6, 8, 7, 8}, {1536, 9, 6, 7, 6, 6}, {2048, 8, 5, 6, 5, 5}};
+    int i = 0;
+    while (cols > F[i].cols) i++;
+    if (solo) return F[i].solo;
+    if (rows <= 4096) return F[i].one;
+    if ((rows - 1) % 8192 + 1 > 6144) return F[i].full;
+    return rows <= 8192 ? F[i].two : F[i].more;
+}
+
+bool f4n_mf(int rows, int cols, int blk_r, int blk_c, int nt)
+{
+    const bool bytes = blk_r != 1 || blk_c != 32 || cols % 128 != 0;
+    return nt >= f4n_from(rows, cols) + bytes;
 }
 
 } // namespace
@@ -264,7 +292,7 @@ int dsv4_fp4_gemv_n_launch(float *y, const float *x, const uint8_t *W, const uin
     }
     const int sc = (cols + blk_c - 1) / blk_c;
     const int ch = cols >> 5;
-    if (f4n_mf(rows, cols, nt)) {
+    if (f4n_mf(rows, cols, blk_r, blk_c, nt)) {
         Dsv4BatchMf b;
         b.fmt = 3; b.y = y; b.x = x; b.W = W; b.S = S;
         b.rows = rows; b.cols = cols; b.nt = nt;

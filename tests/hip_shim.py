@@ -1,7 +1,7 @@
 """A HIP runtime for CPU tests of the library's host code: the calls that
 libdsv4_gpu.so makes to bring itself up and to launch, replaced by ones that
 allocate host memory and launch nothing. A launch can be made to fail, and the
-second launch's second argument is kept. `run` starts a child process with it
+first launch's kernel and the second's second argument are kept. `run` starts a child process with it
 in place; the child sees no device, so nothing runs on a GPU wherever the test
 does. In the child `shim` is this library and `L` the backend."""
 import os
@@ -19,15 +19,35 @@ SOURCE = r"""
 typedef struct { unsigned x, y, z; } D3;
 static int launches, fail_at = -1, last, frees, capturing;
 static void *arg1;
+static const void *first;
+static struct { const void *f; const char *name; } *kernels;
+static int n_kernels;
 /* launch number `at` of the next call fails (-1: none); its stream is or is
  * not being captured */
 void shim_reset(int at, int cap) { launches = 0; last = 0; arg1 = NULL; fail_at = at; capturing = cap; }
 int shim_launches(void) { return launches; }
 int shim_frees(void) { return frees; }
 void *shim_arg1(void) { return arg1; }
+/* the mangled name of the call's first kernel */
+const char *shim_kernel(void)
+{
+    for (int i = 0; i < n_kernels; i++)
+        if (kernels[i].f == first) return kernels[i].name;
+    return "";
+}
+void __hipRegisterFunction(void **m, const void *f, char *d, const char *name, unsigned t, void *a,
+                           void *b, void *c, void *e, int *w)
+{
+    (void)m; (void)d; (void)t; (void)a; (void)b; (void)c; (void)e; (void)w;
+    if ((n_kernels & 255) == 0)
+        kernels = realloc(kernels, (n_kernels + 256) * sizeof *kernels);
+    kernels[n_kernels].f = f;
+    kernels[n_kernels++].name = strdup(name);
+}
 int hipLaunchKernel(const void *f, D3 g, D3 b, void **a, size_t l, void *s)
 {
-    (void)f; (void)g; (void)b; (void)l; (void)s;
+    (void)g; (void)b; (void)l; (void)s;
+    if (launches == 0) first = f;
     if (launches == 1) arg1 = *(void **)a[1];
     if (launches++ == fail_at) { last = 719; return 719; }
     return 0;
@@ -73,6 +93,7 @@ import sys
 import numpy as np
 shim = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 shim.shim_arg1.restype = ctypes.c_void_p
+shim.shim_kernel.restype = ctypes.c_char_p
 import common
 D = common.load_pkg()
 L = D.lib()

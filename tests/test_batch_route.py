@@ -1,0 +1,43 @@
+"""Which kernel a batched FP4 call takes, at shapes where the two were timed (us,
+matrix core / VALU kernel), on both sides of the rule's lines. CPU only."""
+import hip_shim
+
+CHILD = r"""
+buf = np.zeros(1 << 12, np.uint8)
+a = (buf.ctypes.data + 255) // 256 * 256                     # nothing reads it
+assert L.dsv4_gpu_init() == 0
+def route(call):
+    shim.shim_reset(-1, 0)
+    assert call() == 0
+    n = shim.shim_kernel()
+    assert (b"k_batch_mf" in n) != (b"gemv_n" in n), n
+    return b"k_batch_mf" in n
+for rows, cols, nt, mf in SHAPES:
+    got = route(lambda: CALL(rows, cols, nt))
+    assert got == mf, (rows, cols, nt, got)
+print("ok")
+"""
+
+FP4 = [
+    # up to 2048 columns, one VALU workgroup a CU: 6.0 / 4.4, 7.6 / 5.0, 7.9 /
+    # 6.5, 8.2 / 8.5, 4.5 / 4.2, 4.5 / 4.8
+    (1024, 1024, 4, False), (1024, 1536, 4, False), (64, 1536, 7, False), (2048, 2048, 8, True),
+    (2048, 128, 5, False), (2048, 128, 7, True),
+    # one tile a CU: 5.8 / 4.7, 5.8 / 6.2, 8.2 / 8.8
+    (4096, 512, 4, False), (4096, 512, 7, True), (4096, 2048, 5, True),
+    # a round of two a CU begun: 11.1 / 8.3, 10.7 / 7.1, 11.5 / 12.9
+    (6144, 1536, 4, False), (6144, 1024, 4, False), (6144, 2048, 6, True),
+    # ... and full: 10.6 / 9.1, 10.7 / 11.3, 18.5 / 12.4, 18.6 / 19.3
+    (8192, 1024, 5, False), (8192, 1024, 7, True), (16384, 1024, 4, False),
+    (16384, 1024, 7, True),
+    # above 2048 columns: 15.0 / 12.5, 11.1 / 9.9, 12.5 / 14.6, 15.6 / 18.8
+    (1024, 7168, 4, False), (2048, 3584, 4, False), (1024, 4096, 5, True), (2048, 7168, 4, True),
+    # scales byte by byte: 12.5 / 11.8, 11.3 / 6.9
+    (512, 4128, 5, False), (6144, 1056, 4, False),
+]
+
+
+def test_fp4(tmp_path):
+    child = CHILD.replace("SHAPES", repr(FP4)).replace(
+        "CALL(rows, cols, nt)", "L.dsv4_gpu_fp4_gemv_n_d(a, a, a, a, rows, cols, 1, 32, nt, None)")
+    assert hip_shim.run(tmp_path, child).endswith("ok\n")
