@@ -167,15 +167,16 @@ void b16_launch(const B16Geom &g, float *y, const float *x, const uint16_t *W, i
 /* From how many tokens the batch runs on the f32 matrix core
  * (dsv4_batch_mf.hip, the same bits): its time hardly depends on the tokens
  * of a tile of 16, k_bf16_gemv_n's is a few us plus so much per token (us,
- * matrix core / k_bf16_gemv_n: 4096x1024 at 2 tokens 5.5 / 5.3, at 3 5.4 /
- * 6.2; 256x4096 at 5 10.5 / 9.4, at 6 10.5 / 10.9; 16384x2048 at 5 24.2 /
- * 23.4, at 6 24.3 / 25.8; 256x7168 at 7 15.9 / 15.5, at 9 15.8 / 19.1;
- * 64x16384 at 8 31.5 / 29.3, at 9 31.6 / 32.5; 1024x4096 at 48 tokens 11.3 /
- * 65.9). */
+ * matrix core / k_bf16_gemv_n: 1024x256 at 2 tokens 3.9 / 3.7, at 3 4.0 /
+ * 4.4; 64x1024 at 3 5.4 / 5.0, at 4 5.4 / 5.9; 256x4096 at 5 10.5 / 9.4, at
+ * 6 10.5 / 10.9; 16384x2048 at 5 24.2 / 23.4, at 6 24.3 / 25.8; 256x7168 at
+ * 7 15.9 / 15.5, at 9 15.8 / 19.1; 64x16384 at 8 31.5 / 29.3, at 9 31.6 /
+ * 32.5; 1024x4096 at 48 tokens 11.3 / 65.9). */
 bool b16n_mf(const B16Geom &g, int rows, int nt)
 {
     const long long tiles = (long long)((rows + 15) / 16) * ((nt + 15) / 16);
-    return g.tc >= 4 && nt >= (g.ch <= 128 && tiles <= 256 ? 3 : g.ch <= 512 ? 6 : 9);
+    const int from = g.ch <= 128 && tiles <= 256 ? (g.ch <= 32 ? 3 : 4) : g.ch <= 512 ? 6 : 9;
+    return g.tc >= 4 && nt >= from;
 }
 
 int b16_dispatch(const B16Geom &g, float *y, const float *x, const uint16_t *W, int rows,

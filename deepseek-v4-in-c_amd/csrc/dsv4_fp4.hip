@@ -252,9 +252,10 @@ void f4n_launch(float *y, const float *x, const uint8_t *W, const uint8_t *S, in
  *     10.5; 8192x1024 at 6 10.7 / 10.3, at 7 10.7 / 11.3; 10240x512 at 9
  *     13.6 / 13.1; 8192x2048 at 4 11.6 / 11.7.
  * Of 4620 shapes of 16 to 16384 rows, 128 to 16384 columns and 2 to 12 tokens
- * none is more than 5 % slower than on k_fp4_gemv_n. Where the tile reads its scales byte by byte (not 1x32 blocks, or a ragged last
- * step) it starts a token later (64x8192 of 32x64 blocks at 5 tokens 18.4 /
- * 17.2, 512x4128 at 5 12.5 / 11.8). */
+ * none is more than 5 % slower than on k_fp4_gemv_n. Where the tile reads its
+ * scales byte by byte (not 1x32 blocks, or a ragged last step) it starts a
+ * token later (64x8192 of 32x64 blocks at 5 tokens 18.4 / 17.2, 512x4128 at 5
+ * 12.5 / 11.8). */
 int f4n_from(int rows, int cols)
 {
     const bool solo = rows <= (cols > 4096 ? 1024 : 2048);     /* a workgroup a CU */

@@ -1,5 +1,7 @@
-"""Which kernel a batched FP4 call takes, at shapes where the two were timed (us,
+"""Which kernel a batched FP4 or BF16 call takes, at shapes where the two were timed (us,
 matrix core / VALU kernel), on both sides of the rule's lines. CPU only."""
+import pytest
+
 import hip_shim
 
 CHILD = r"""
@@ -36,8 +38,17 @@ FP4 = [
     (512, 4128, 5, False), (6144, 1056, 4, False),
 ]
 
+BF16 = [
+    # up to 256 columns; up to 1024: 5.5 / 5.0, 5.7 / 5.4, 5.4 / 5.9; above
+    (1024, 256, 2, False), (1024, 256, 3, True),
+    (64, 1024, 3, False), (1024, 1024, 3, False), (64, 512, 3, False), (64, 1024, 4, True),
+    (256, 4096, 5, False), (256, 4096, 6, True), (256, 7168, 8, False), (256, 7168, 9, True),
+]
 
-def test_fp4(tmp_path):
-    child = CHILD.replace("SHAPES", repr(FP4)).replace(
-        "CALL(rows, cols, nt)", "L.dsv4_gpu_fp4_gemv_n_d(a, a, a, a, rows, cols, 1, 32, nt, None)")
+
+@pytest.mark.parametrize("shapes,call", [
+    (FP4, "L.dsv4_gpu_fp4_gemv_n_d(a, a, a, a, rows, cols, 1, 32, nt, None)"),
+    (BF16, "L.dsv4_gpu_bf16_gemv_n_d(a, a, a, rows, cols, nt, None)")], ids=["fp4", "bf16"])
+def test_route(tmp_path, shapes, call):
+    child = CHILD.replace("SHAPES", repr(shapes)).replace("CALL(rows, cols, nt)", call)
     assert hip_shim.run(tmp_path, child).endswith("ok\n")
