@@ -1059,21 +1059,25 @@ int dsv4_gpu_moe_fp4_n(float *out, const float *x, int layer, const int *idx,
     size_t end;
     if (stage_push(s, &end) != 0) return -1;
     /* With the routing in hand: two tokens whose (token, k) pairs barely share
-     * experts (distinct experts above 9 in 10 pairs) of C3's size or more go
-     * one by one through the single-token kernels, whose 2 x 8 experts take
-     * 76.1 us at 7168 x 2048 against 79.1 batched. Smaller experts and more
-     * tokens are faster batched with every expert distinct (us, batched /
-     * token by token: 7168 x 2048 top 8, 3 tokens 109.8 / 115.4, 4 tokens
-     * 143.9 / 153.9; 4096 x 2048 top 6, 2 tokens 47.4 / 60.2). Both give
-     * every token the same bits. DSV4_GPU_MOEN_TOKENWISE: 1 always token by
-     * token, 0 never. */
+     * experts (distinct experts above 9 in 10 pairs) go one by one through the
+     * single-token kernels where those are at their best: both their unit
+     * loops unrolled (hidden 7168, inter 2048) and their 64 gate/up workgroups
+     * per expert in rounds of 256 CUs at least 3/4 full. Else the batched form
+     * is the faster or as fast, with every expert distinct (us, the host call
+     * batched / token by token: 7168 x 2048, 2 tokens, top 8 95.8 / 93.1, top
+     * 7 91.3 / 88.6, top 12 123.4 / 121.4; top 6 81.7 / 86.2, top 10 108.0 /
+     * 115.9, top 2 51.7 / 61.7; 3 tokens of top 8 123.9 / 130.2; 8192 x 2048
+     * top 8 112.9 / 113.0, top 6 92.1 / 102.2; 7680 x 2048 104.0 / 105.2; 6144
+     * x 2048 91.1 / 93.4; 4096 x 2048 top 6 63.7 / 75.6). Both give every
+     * token the same bits. DSV4_GPU_MOEN_TOKENWISE: 1 always token by token,
+     * 0 never. */
     int tokenwise = moen_tokenwise_env();
     if (tokenwise < 0) {
         std::vector<int> seen(idx, idx + (size_t)nt * topk);
         std::sort(seen.begin(), seen.end());
         const size_t distinct = std::unique(seen.begin(), seen.end()) - seen.begin();
-        tokenwise = nt == 2 && (size_t)hidden * inter >= (size_t)7168 * 2048 &&
-                    10 * distinct > 9 * (size_t)nt * topk;
+        tokenwise = nt == 2 && hidden == 7168 && inter == 2048 && topk > 3 &&
+                    (topk % 4 == 0 || topk % 4 == 3) && 10 * distinct > 9 * (size_t)nt * topk;
     }
     if (tokenwise) {
         for (int t = 0; t < nt; t++)

@@ -1,9 +1,10 @@
 """A HIP runtime for CPU tests of the library's host code: the calls that
 libdsv4_gpu.so makes to bring itself up and to launch, replaced by ones that
 allocate host memory and launch nothing. A launch can be made to fail, and the
-first launch's kernel and the second's second argument are kept. `run` starts a child process with it
-in place; the child sees no device, so nothing runs on a GPU wherever the test
-does. In the child `shim` is this library and `L` the backend."""
+first eight kernels and the second launch's second argument are kept. `run`
+starts a child process with it in place; the child sees no device, so nothing
+runs on a GPU wherever the test does. In the child `shim` is this library and
+`L` the backend."""
 import os
 import shutil
 import subprocess
@@ -19,7 +20,7 @@ SOURCE = r"""
 typedef struct { unsigned x, y, z; } D3;
 static int launches, fail_at = -1, last, frees, capturing;
 static void *arg1;
-static const void *first;
+static const void *ran[8];
 static struct { const void *f; const char *name; } *kernels;
 static int n_kernels;
 /* launch number `at` of the next call fails (-1: none); its stream is or is
@@ -28,11 +29,11 @@ void shim_reset(int at, int cap) { launches = 0; last = 0; arg1 = NULL; fail_at 
 int shim_launches(void) { return launches; }
 int shim_frees(void) { return frees; }
 void *shim_arg1(void) { return arg1; }
-/* the mangled name of the call's first kernel */
-const char *shim_kernel(void)
+/* the mangled name of the call's kernel number k */
+const char *shim_kernel(int k)
 {
     for (int i = 0; i < n_kernels; i++)
-        if (kernels[i].f == first) return kernels[i].name;
+        if (k < launches && k < 8 && kernels[i].f == ran[k]) return kernels[i].name;
     return "";
 }
 void __hipRegisterFunction(void **m, const void *f, char *d, const char *name, unsigned t, void *a,
@@ -47,7 +48,7 @@ void __hipRegisterFunction(void **m, const void *f, char *d, const char *name, u
 int hipLaunchKernel(const void *f, D3 g, D3 b, void **a, size_t l, void *s)
 {
     (void)g; (void)b; (void)l; (void)s;
-    if (launches == 0) first = f;
+    if (launches < 8) ran[launches] = f;
     if (launches == 1) arg1 = *(void **)a[1];
     if (launches++ == fail_at) { last = 719; return 719; }
     return 0;
@@ -74,6 +75,16 @@ int hipDeviceSynchronize(void) { return 0; }
 int hipMalloc(void **p, size_t n) { *p = malloc(n); return *p ? 0 : 2; }
 int hipMemset(void *p, int v, size_t n) { memset(p, v, n); return 0; }
 int hipFree(void *p) { (void)p; frees++; return 0; }
+int hipHostMalloc(void **p, size_t n, unsigned fl) { (void)fl; *p = malloc(n); return *p ? 0 : 2; }
+int hipHostGetDevicePointer(void **d, void *h, unsigned fl) { (void)fl; *d = h; return 0; }
+int hipMemcpy(void *d, const void *s, size_t n, int k) { (void)k; memcpy(d, s, n); return 0; }
+int hipMemcpyAsync(void *d, const void *s, size_t n, int k, void *st)
+{
+    (void)k; (void)st;
+    memcpy(d, s, n);
+    return 0;
+}
+int hipStreamSynchronize(void *st) { (void)st; return 0; }
 int hipStreamIsCapturing(void *s, int *st) { (void)s; *st = capturing; return 0; }
 int hipDeviceGetAttribute(int *v, int attr, int d)
 {
@@ -83,7 +94,7 @@ int hipDeviceGetAttribute(int *v, int attr, int d)
 }
 int hipFuncGetAttributes(void *a, const void *f) { (void)a; (void)f; return 1; }
 int hipFuncSetAttribute(const void *f, int at, int v) { (void)f; (void)at; (void)v; return 0; }
-int hipGetDevicePropertiesR0600(void *p, int d) { (void)d; memset(p, 0, 256); return 0; }
+int hipGetDevicePropertiesR0600(void *p, int d) { (void)d; memset(p, 0, PROP); return 0; }
 """
 
 # before torch and the backend, whose calls then find it first
@@ -103,7 +114,11 @@ _CU = r"""
 #include <hip/hip_runtime_api.h>
 #include <cstdio>
 static_assert(sizeof(hipDeviceAttribute_t) == sizeof(int), "");
-int main() { printf("%d", (int)hipDeviceAttributeMultiprocessorCount); }
+int main()
+{
+    printf("-DATTR_CU=%d -DPROP=%d", (int)hipDeviceAttributeMultiprocessorCount,
+           (int)sizeof(hipDeviceProp_t));
+}
 """
 
 
@@ -118,9 +133,8 @@ def run(tmp_path, child, env=None):
     with open(src, "w") as f:
         f.write(SOURCE)
     subprocess.run(["g++", "-D__HIP_PLATFORM_AMD__", "-w", "-I", hip, cu, "-o", exe], check=True)
-    attr = subprocess.run([exe], capture_output=True, text=True, check=True).stdout
-    subprocess.run(["gcc", "-shared", "-fPIC", "-Wall", "-Werror", "-DATTR_CU=" + attr, src,
-                    "-o", lib], check=True)
+    defs = subprocess.run([exe], capture_output=True, text=True, check=True).stdout.split()
+    subprocess.run(["gcc", "-shared", "-fPIC", "-Wall", "-Werror"] + defs + [src, "-o", lib], check=True)
     e = dict(os.environ, HIP_VISIBLE_DEVICES="-1", **(env or {}))
     e["PYTHONPATH"] = os.pathsep.join([os.path.join(common.ROOT, "tests"), common.ROOT,
                                        e.get("PYTHONPATH", "")])

@@ -1,5 +1,6 @@
-"""Which kernel a batched FP4 or BF16 call takes, at shapes where the two were timed (us,
-matrix core / VALU kernel), on both sides of the rule's lines. CPU only."""
+"""Which kernels a batched call takes, at shapes where both were timed, on both
+sides of the rules' lines: FP4 and BF16 (us, matrix core / VALU kernel) and the
+routed experts' host call (batched / token by token). CPU only."""
 import pytest
 
 import hip_shim
@@ -11,7 +12,7 @@ assert L.dsv4_gpu_init() == 0
 def route(call):
     shim.shim_reset(-1, 0)
     assert call() == 0
-    n = shim.shim_kernel()
+    n = shim.shim_kernel(0)
     assert (b"k_batch_mf" in n) != (b"gemv_n" in n), n
     return b"k_batch_mf" in n
 for rows, cols, nt, mf in SHAPES:
@@ -52,3 +53,43 @@ BF16 = [
 def test_route(tmp_path, shapes, call):
     child = CHILD.replace("SHAPES", repr(shapes)).replace("CALL(rows, cols, nt)", call)
     assert hip_shim.run(tmp_path, child).endswith("ok\n")
+
+
+MOE = r"""
+assert L.dsv4_gpu_init() == 0
+def batched(layer, hidden, inter, topk, nt, distinct):
+    if not L.dsv4_gpu_has_expert(layer, 0):
+        for e in range(64):                                  # nothing reads them
+            q = lambda o, r, c: D.DSV4QMat(4096 * (1 + o), 4096 * (4 + o), D.WFP4, r, c, 1, 32)
+            ew = D.DSV4ExpertW(q(0, inter, hidden), q(1, inter, hidden), q(2, hidden, inter))
+            assert L.dsv4_gpu_bind_expert_d(layer, e, ctypes.byref(ew)) == 0
+    idx = np.arange(nt * topk, dtype=np.int32) % distinct
+    w = np.ones(nt * topk, np.float32)
+    x = np.zeros((nt, hidden), np.float32)
+    out = np.empty((nt, hidden), np.float32)
+    shim.shim_reset(-1, 0)
+    assert L.dsv4_gpu_moe_fp4_n(out.ctypes.data, x.ctypes.data, layer, idx.ctypes.data,
+                                w.ctypes.data, nt, topk, hidden, inter, 10.0) == 0
+    return any(b"k_mn_prepare" in shim.shim_kernel(i) for i in range(shim.shim_launches()))
+for layer, hidden, inter, topk, nt, distinct, want in SHAPES:
+    assert batched(layer, hidden, inter, topk, nt, distinct) == want, (hidden, inter, topk, nt)
+print("ok")
+"""
+
+# layer, hidden, inter, topk, nt, distinct experts, batched: 95.8 / 93.1, 91.3 /
+# 88.6, 81.7 / 86.2, 108.0 / 115.9, 51.7 / 61.7, 125.6 / 131.3, shared experts,
+# 112.9 / 113.0, 92.1 / 102.2, 91.1 / 93.4
+MOE_SHAPES = [
+    (0, 7168, 2048, 8, 2, 16, False), (0, 7168, 2048, 7, 2, 14, False),
+    (0, 7168, 2048, 6, 2, 12, True), (0, 7168, 2048, 10, 2, 20, True),
+    (0, 7168, 2048, 2, 2, 4, True), (0, 7168, 2048, 8, 3, 24, True),
+    (0, 7168, 2048, 8, 2, 12, True), (1, 8192, 2048, 8, 2, 16, True),
+    (1, 8192, 2048, 6, 2, 12, True), (2, 6144, 2048, 8, 2, 16, True),
+]
+
+
+@pytest.mark.parametrize("mode", [None, "0", "1"])
+def test_route_moe(tmp_path, mode):
+    shapes = [s if mode is None else s[:-1] + (mode == "0",) for s in MOE_SHAPES]
+    env = {} if mode is None else {"DSV4_GPU_MOEN_TOKENWISE": mode}
+    assert hip_shim.run(tmp_path, MOE.replace("SHAPES", repr(shapes)), env).endswith("ok\n")

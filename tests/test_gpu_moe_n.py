@@ -90,7 +90,9 @@ def test_moe_n_c3_shape(gpu, dsv4, nt):
 
 def test_moe_n_one_expert_set_for_every_token(gpu, dsv4):
     """64 tokens that all ask for the same 8 experts: 64 pairs per expert, so
-    each expert runs 13 passes of 5 pairs over its (once-streamed) weights."""
+    each expert runs 7 passes of up to 10 pairs over its weights. (The ids lie
+    below 32, so 512 pairs are more than five per table entry: two column
+    tiles a pass.)"""
     rng, table = _setup(dsv4, 6, 7168, 2048, 8, 7)
     IDX, W, X = _batch(rng, table, 64, 8, 7168, same=True)
     _check(dsv4, 6, table, IDX, W, X, 7168, 2048, 10.0, oracle_tokens=[0, 33, 63])
@@ -106,17 +108,22 @@ def test_moe_n_other_shapes(gpu, dsv4, hidden, inter, topk, nt, limit):
     _check(dsv4, 7, table, IDX, W, X, hidden, inter, limit)
 
 
+@pytest.mark.parametrize("layer,hidden,inter,topk,nt", [
+    (11, 2048, 1024, 8, 4), (12, 7168, 2048, 8, 2), (13, 7168, 2048, 6, 2)])
 @pytest.mark.parametrize("mode", ["auto", "0", "1"])
-def test_moe_n_tokenwise_rule(gpu, dsv4, monkeypatch, mode):
-    """Pairs that barely share experts (4 tokens x top-8 drawn from 64
-    experts): the host-buffer call then runs the tokens one by one through
-    the single-token kernels (auto, or DSV4_GPU_MOEN_TOKENWISE=1); =0 keeps
-    the batched kernels. Every mode gives each token its single-token bits."""
+def test_moe_n_tokenwise_rule(gpu, dsv4, monkeypatch, mode, layer, hidden, inter, topk, nt):
+    """Pairs that barely share experts: the host-buffer call runs the tokens
+    one by one through the single-token kernels (DSV4_GPU_MOEN_TOKENWISE=1;
+    auto: two tokens x top-8 at 7168 x 2048 only) or batched (=0; auto: the
+    others, tests/test_batch_route.py). Every mode gives each token its
+    single-token bits."""
     if mode != "auto":
         monkeypatch.setenv("DSV4_GPU_MOEN_TOKENWISE", mode)
-    rng, table = _setup(dsv4, 11, 2048, 1024, 64, 13)
-    IDX, W, X = _batch(rng, table, 4, 8, 2048)
-    _check(dsv4, 11, table, IDX, W, X, 2048, 1024, 10.0)
+    rng, table = _setup(dsv4, layer, hidden, inter, 64 if nt > 2 else 16, 13)
+    IDX, W, X = _batch(rng, table, nt, topk, hidden)
+    if nt == 2:
+        IDX[:] = rng.permutation(np.array(sorted(table), np.int32))[:nt * topk].reshape(nt, topk)
+    _check(dsv4, layer, table, IDX, W, X, hidden, inter, 10.0)
 
 
 @pytest.mark.parametrize("form", ["0", "1"])
