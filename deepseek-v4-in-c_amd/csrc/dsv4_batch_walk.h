@@ -39,14 +39,14 @@ struct MfWalk {
     }
 };
 
-/* The steps of such a wave; nch = ceil(ch / tc). */
+/* The steps of such a wave; nch = ceil(ch / tc), so only the last pass of a
+ * group in the row can lie outside it. No loop: the first copies wait for
+ * this (1024x4096 BF16 at 48 tokens 10.81 us with a loop over the groups). */
 DSV4_HD int mf_steps(int j0, int L, int tc, int ch, int nch)
 {
-    const int groups = L >> 2, in_row = (ch - j0 + 3) >> 2;
-    const int live = j0 < ch ? (groups < in_row ? groups : in_row) : 0;
-    int steps = 0;
-    for (int u = 0; u < live; u++) steps += nch - (j0 + 4 * u + (nch - 1) * tc < ch ? 0 : 1);
-    return steps;
+    const int groups = L >> 2, rest = ch - (nch - 1) * tc;     /* the last pass's chunks */
+    const int in_row = j0 < ch ? (ch - j0 + 3) >> 2 : 0, last = j0 < rest ? (rest - j0 + 3) >> 2 : 0;
+    return (groups < in_row ? groups : in_row) * (nch - 1) + (groups < last ? groups : last);
 }
 
 #endif
