@@ -171,11 +171,15 @@ void b16_launch(const B16Geom &g, float *y, const float *x, const uint16_t *W, i
  * 4.4; 64x1024 at 3 5.4 / 5.0, at 4 5.4 / 5.9; 256x4096 at 5 10.5 / 9.4, at
  * 6 10.5 / 10.9; 16384x2048 at 5 24.2 / 23.4, at 6 24.3 / 25.8; 256x7168 at
  * 7 15.9 / 15.5, at 9 15.8 / 19.1; 64x16384 at 8 31.5 / 29.3, at 9 31.6 /
- * 32.5; 1024x4096 at 48 tokens 11.3 / 65.9). */
+ * 32.5; 1024x4096 at 48 tokens 11.3 / 65.9). Where the widest rows end inside
+ * a step, whose copies then clamp their columns, a tile is a fifth slower, and
+ * up to 1024 rows the VALU keeps more tokens (512x15352 at 9 40.3 / 33.1, at
+ * 12 43.4 / 42.8; 1100x15352 at 9 41.0 / 64.7). */
 bool b16n_mf(const B16Geom &g, int rows, int nt)
 {
     const long long tiles = (long long)((rows + 15) / 16) * ((nt + 15) / 16);
-    const int from = g.ch <= 128 && tiles <= 256 ? (g.ch <= 32 ? 3 : 4) : g.ch <= 512 ? 6 : 9;
+    const int from = g.ch <= 128 && tiles <= 256 ? (g.ch <= 32 ? 3 : 4) : g.ch <= 512 ? 6
+                   : g.ch > 1536 && g.ch % 4 != 0 && rows <= 1024 ? 12 : 9;
     return g.tc >= 4 && nt >= from;
 }
 

@@ -44,6 +44,10 @@ BF16 = [
     (1024, 256, 2, False), (1024, 256, 3, True),
     (64, 1024, 3, False), (1024, 1024, 3, False), (64, 512, 3, False), (64, 1024, 4, True),
     (256, 4096, 5, False), (256, 4096, 6, True), (256, 7168, 8, False), (256, 7168, 9, True),
+    # the widest, ending inside a step or not: 40.3 / 33.1,
+    # 43.4 / 42.8, 41.0 / 64.7, 32.1 / 33.0
+    (512, 15352, 9, False), (512, 15352, 12, True), (1100, 15352, 9, True),
+    (512, 15360, 9, True),
 ]
 
 

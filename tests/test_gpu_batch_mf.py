@@ -81,7 +81,8 @@ def test_fp8_blockings(gpu, dsv4, blk_r, blk_c):
 
 @pytest.mark.parametrize("rows,cols,nt", [
     (1, 32, 9), (17, 40, 9), (16, 512, 16), (31, 1048, 20), (300, 4096, 48), (1030, 4096, 64),
-    (9000, 1024, 33), (40, 7168, 33), (33, 8200, 10), (20, 12296, 9), (18, 16384, 17)])
+    (9000, 1024, 33), (40, 7168, 33), (33, 8200, 10), (20, 12296, 9), (20, 12296, 12),
+    (18, 16384, 17)])
 def test_bf16(gpu, dsv4, rows, cols, nt):
     rng = np.random.default_rng(rows + cols + nt)
     W = common.bf16_matrix(rng, (rows, cols), 0.02)
