@@ -870,13 +870,6 @@ void launch_gemv_nl_nch(const Fp8Geom &g, float *y, const float *x, const uint8_
  * batch, unsplit. */
 int mf_slots() { return env_int("DSV4_GPU_MFN_L", 0); }
 
-bool mf_takes(const Fp8Geom &g, int rows, int blk_r, int nt)
-{
-    const int from = g.tc != 192 ? 5 : rows <= 256 ? 11 : rows <= 512 ? 9 : 8;
-    return env_int("DSV4_GPU_FP8_MFN", 1) != 0 && nt >= 2 && g.tc >= 4 && (blk_r & 15) == 0 &&
-           (mf_slots() != 0 || nt >= from);
-}
-
 int mf_split(const Fp8Geom &g, int rows, int nt)
 {
     const long long tiles = (long long)((rows + 15) / 16) * ((nt + 15) / 16);
@@ -889,6 +882,36 @@ int mf_split(const Fp8Geom &g, int rows, int nt)
     return tiles * 4 <= cu ? 4 : tiles * 2 <= cu ? 2 : 1;
 }
 
+/* the most LDS k_fp8_gemv_nl takes for a block of tokens' x */
+size_t nl_cap() { return dsv4_lds_limit() - 2048; }
+
+/* From how many tokens. Where tiles would be split but the call has no place for
+ * their part sums (a captured one, say), a whole tile's chain is twice or four
+ * times as long, and the VALU keeps more tokens (us, whole tiles / VALU):
+ *   - 128 threads a row: 512x6144 at 5 tokens 14.8 / 13.2, at 7 14.8 / 14.2;
+ *     where k_fp8_gemv_nl holds eight tokens of x, 512x4112 at 8 1.16 times
+ *     the VALU's, at 9 0.77;
+ *   - 192: 64x10240 at 12 21.2 / 13.4, 512x12288 at 12 24.7 / 22.7, at 16
+ *     25.2 / 27.9, 1024x12288 at 8 24.6 / 30.3;
+ *   - 256: 512x14336 at 8 27.2 / 24.9, at 9 27.6 / 28.9; 512x16384 at 9 30.8
+ *     / 29.9; of 1360 rows on from 5. */
+int mf_from(const Fp8Geom &g, int rows, int cols, bool whole)
+{
+    if (g.tc == 192) {
+        if (whole) return rows <= 256 ? 21 : rows <= 512 ? 15 : rows <= 768 ? 10 : 8;
+        return rows <= 256 ? 11 : rows <= 512 ? 9 : 8;
+    }
+    if (whole && g.tc == 128) return 8 * sizeof(float) * (size_t)cols <= nl_cap() ? 9 : 7;
+    if (whole && g.tc == 256 && rows <= 1024) return cols > 15360 ? 10 : 9;
+    return 5;
+}
+
+bool mf_takes(const Fp8Geom &g, int rows, int cols, int blk_r, int nt, bool whole)
+{
+    return env_int("DSV4_GPU_FP8_MFN", 1) != 0 && nt >= 2 && g.tc >= 4 && (blk_r & 15) == 0 &&
+           (mf_slots() != 0 || nt >= mf_from(g, rows, cols, whole));
+}
+
 /* 0; -1 where the f32 matrix-core form's launch failed, whose error it has
  * taken (a failed launch of the others is still there for the caller to get) */
 template <int SF>
@@ -896,13 +919,14 @@ int launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
                   const void *S, int rows, int cols, int sc, int blk_r,
                   int blk_c, int nt, hipStream_t st, void *scratch)
 {
-    if (mf_takes(g, rows, blk_r, nt)) {
+    const int split = mf_split(g, rows, nt);
+    if (mf_takes(g, rows, cols, blk_r, nt, split > 1 && !scratch)) {
         Dsv4BatchMf b;
         b.fmt = SF; b.y = y; b.x = x; b.W = W; b.S = S;
         b.rows = rows; b.cols = cols; b.nt = nt;
         b.tc = g.tc; b.sc = sc; b.blk_r = blk_r; b.blk_c = blk_c;
         b.slots = mf_slots();
-        b.split = mf_split(g, rows, nt);
+        b.split = split;
         b.part = (float *)scratch;
         const int rc = dsv4_batch_mf_launch(b, st);
         if (rc <= 0) return rc;
@@ -911,7 +935,7 @@ int launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
      * and the tokens fill (8 x 4096, 4 x 7168, 2 x 16384 columns); three
      * tokens take one block of four rather than two of two (us, 7168x7168 31.9
      * -> 24.0, 1536x7168 11.3 -> 10.1) */
-    const size_t cap = dsv4_lds_limit() - 2048;
+    const size_t cap = nl_cap();
     if (nt >= 2 && (((uintptr_t)x) & 15) == 0 && g.tc <= 256 && 512 % g.tc == 0) {
         const size_t row4 = sizeof(float) * (size_t)cols;
         if (nt >= 8 && 8 * row4 <= cap) { launch_gemv_nl_nch<SF, 8>(g, y, x, W, S, rows, cols, sc, blk_r, blk_c, nt, st); return 0; }

@@ -162,11 +162,12 @@ int scratch_reserve(Scratch &s, size_t bytes)
  * per stream: calls on one stream follow each other, so a slot's next call
  * comes after its last join, and calls on different streams never meet in one.
  * A few streams' slots, allocated by dsv4_gpu_init and never moved or handed on
- * until dsv4_gpu_shutdown. A call without a slot takes the unsplit form, which
- * needs none and gives the same bits (1536x7168 at 13 tokens 15.4 us for 13.0):
- * on a stream that comes after SPLIT_SLOTS others, and on hipStreamPerThread,
- * one name for several streams. So does a call under capture, whose graph may
- * be replayed on any stream, beside calls on the one it was captured on. */
+ * until dsv4_gpu_shutdown. A call without a slot takes whole tiles, which need
+ * none, or the VALU where that is then the faster (mf_from), with the same bits
+ * (1536x7168 at 13 tokens 15.4 us for 13.0): on a stream that comes after
+ * SPLIT_SLOTS others, and on hipStreamPerThread, one name for several streams.
+ * So does a call under capture, whose graph may be replayed on any stream,
+ * beside calls on the one it was captured on. */
 constexpr int SPLIT_SLOTS = 8;
 struct SplitPool {
     std::mutex mu;

@@ -1,6 +1,7 @@
 """Which kernels a batched call takes, at shapes where both were timed, on both
-sides of the rules' lines: FP4 and BF16 (us, matrix core / VALU kernel) and the
-routed experts' host call (batched / token by token). CPU only."""
+sides of the rules' lines: FP4 and BF16 (us, matrix core / VALU kernel), FP8 with
+and without a place for part sums, and the routed experts' host call (batched /
+token by token). CPU only."""
 import pytest
 
 import hip_shim
@@ -9,8 +10,8 @@ CHILD = r"""
 buf = np.zeros(1 << 12, np.uint8)
 a = (buf.ctypes.data + 255) // 256 * 256                     # nothing reads it
 assert L.dsv4_gpu_init() == 0
-def route(call):
-    shim.shim_reset(-1, 0)
+def route(call, capture=0):
+    shim.shim_reset(-1, capture)
     assert call() == 0
     n = shim.shim_kernel(0)
     assert (b"k_batch_mf" in n) != (b"gemv_n" in n), n
@@ -56,6 +57,33 @@ BF16 = [
     (BF16, "L.dsv4_gpu_bf16_gemv_n_d(a, a, a, rows, cols, nt, None)")], ids=["fp4", "bf16"])
 def test_route(tmp_path, shapes, call):
     child = CHILD.replace("SHAPES", repr(shapes)).replace("CALL(rows, cols, nt)", call)
+    assert hip_shim.run(tmp_path, child).endswith("ok\n")
+
+
+FP8_STREAM = CHILD.split("for rows")[0] + r"""
+for rows, cols, nt, eager, captured in SHAPES:
+    for sf in (0, 1):
+        call = lambda: L.dsv4_gpu_fp8_gemv_n_d(a, a, a, a, sf, rows, cols, nt, a)
+        got = route(call), route(call, 1)
+        assert got == (eager, captured), (rows, cols, nt, got)
+print("ok")
+"""
+
+# on a stream with a place for part sums, and captured, where tiles stay whole
+# (us, whole tiles / VALU): 14.8 / 13.2, 14.8 / 14.2, 1.16 and 0.77 times, 21.2 /
+# 13.4, 24.7 / 22.7, 25.2 / 27.9, 27.2 / 24.9, 27.6 / 28.9, 30.8 / 29.9, 11.2 / 15.2
+FP8_SHAPES = [
+    (512, 6144, 5, True, False), (512, 6144, 7, True, True), (512, 4112, 8, True, False),
+    (512, 4112, 9, True, True), (64, 10240, 12, True, False), (512, 12288, 12, True, False),
+    (512, 12288, 16, True, True), (512, 14336, 8, True, False), (512, 14336, 9, True, True),
+    (512, 16384, 9, True, False), (512, 4096, 5, True, True),
+    # tiles that are not split in either: 192 threads a row, 128
+    (3000, 7168, 5, True, True), (2000, 12288, 8, True, True), (2000, 12288, 7, False, False),
+]
+
+
+def test_route_fp8(tmp_path):
+    child = FP8_STREAM.replace("SHAPES", repr(FP8_SHAPES))
     assert hip_shim.run(tmp_path, child).endswith("ok\n")
 
 
