@@ -855,7 +855,11 @@ void launch_gemv_nl_nch(const Fp8Geom &g, float *y, const float *x, const uint8_
  * columns none of 5 tokens or more was slower than before). Rows of 192
  * threads, which k_fp8_gemv_nl does not take: from 8 tokens, few of them from
  * 9 or 11 (64x8208 at 8 tokens 10.5 / 8.2, at 10 10.6 / 10.1; 256x12288 at 9
- * 12.9 / 12.0, at 12 12.9 / 14.6; 512x10240 at 8 13.2 / 12.9).
+ * 12.9 / 12.0, at 12 12.9 / 14.6; 512x10240 at 8 13.2 / 12.9); up to 256 rows
+ * a token later with fp32 scales, which the VALU loads faster, and another
+ * around 10240 columns (fp32 128x8704 at 11 tokens 1.04 times the VALU's, at
+ * 12 0.99; 64x10240 at 11 13.0 / 11.5, at 13 13.4 / 12.8; E8M0 128x10240 at
+ * 11 1.08 times, at 12 1.02).
  *
  * While the tiles leave CUs idle, rows of 4096 columns on are split
  * over 4, 3 or 2 workgroups (a row's 64-slot blocks, or parts of one) that a
@@ -895,21 +899,22 @@ size_t nl_cap() { return dsv4_lds_limit() - 2048; }
  *     25.2 / 27.9, 1024x12288 at 8 24.6 / 30.3;
  *   - 256: 512x14336 at 8 27.2 / 24.9, at 9 27.6 / 28.9; 512x16384 at 9 30.8
  *     / 29.9; of 1360 rows on from 5. */
-int mf_from(const Fp8Geom &g, int rows, int cols, bool whole)
+int mf_from(const Fp8Geom &g, int sfmt, int rows, int cols, bool whole)
 {
     if (g.tc == 192) {
         if (whole) return rows <= 256 ? 21 : rows <= 512 ? 15 : rows <= 768 ? 10 : 8;
-        return rows <= 256 ? 11 : rows <= 512 ? 9 : 8;
+        if (rows <= 256) return 11 + (sfmt != 0) + (cols > 9856 && cols <= 10496);
+        return rows <= 512 ? 9 : 8;
     }
     if (whole && g.tc == 128) return 8 * sizeof(float) * (size_t)cols <= nl_cap() ? 9 : 7;
     if (whole && g.tc == 256 && rows <= 1024) return cols > 15360 ? 10 : 9;
     return 5;
 }
 
-bool mf_takes(const Fp8Geom &g, int rows, int cols, int blk_r, int nt, bool whole)
+bool mf_takes(const Fp8Geom &g, int sfmt, int rows, int cols, int blk_r, int nt, bool whole)
 {
     return env_int("DSV4_GPU_FP8_MFN", 1) != 0 && nt >= 2 && g.tc >= 4 && (blk_r & 15) == 0 &&
-           (mf_slots() != 0 || nt >= mf_from(g, rows, cols, whole));
+           (mf_slots() != 0 || nt >= mf_from(g, sfmt, rows, cols, whole));
 }
 
 /* 0; -1 where the f32 matrix-core form's launch failed, whose error it has
@@ -920,7 +925,7 @@ int launch_gemv_n(const Fp8Geom &g, float *y, const float *x, const uint8_t *W,
                   int blk_c, int nt, hipStream_t st, void *scratch)
 {
     const int split = mf_split(g, rows, nt);
-    if (mf_takes(g, rows, cols, blk_r, nt, split > 1 && !scratch)) {
+    if (mf_takes(g, SF, rows, cols, blk_r, nt, split > 1 && !scratch)) {
         Dsv4BatchMf b;
         b.fmt = SF; b.y = y; b.x = x; b.W = W; b.S = S;
         b.rows = rows; b.cols = cols; b.nt = nt;

@@ -61,7 +61,8 @@ def test_fp8(gpu, dsv4, rows, cols, nt, scales):
 # a tile, 6 (8208: a ragged last group), 3, and the least tokens of few rows
 @pytest.mark.parametrize("scales", ["e8m0", "f32"])
 @pytest.mark.parametrize("rows,cols,nt", [
-    (250, 9216, 11), (500, 10240, 9), (1360, 12288, 33), (4200, 8224, 16), (3000, 9216, 48),
+    (250, 9216, 11), (250, 9216, 12), (500, 10240, 9), (1360, 12288, 33), (4200, 8224, 16),
+    (3000, 9216, 48),
     (2200, 8208, 64), (4100, 9216, 64), (4100, 8208, 64)])
 def test_fp8_192_slots(gpu, dsv4, rows, cols, nt, scales):
     test_fp8(gpu, dsv4, rows, cols, nt, scales)
