@@ -72,6 +72,7 @@ struct LayerExperts {
     size_t dev_cap = 0;
     bool dirty = false;
     int hidden = 0, inter = 0;
+    int resident = 0;                       /* experts in `host`, by layer_sync */
 };
 
 struct Arena {
@@ -434,6 +435,8 @@ int layer_sync(LayerExperts &L)
     }
     HIP_OK(hipMemcpy(L.dev, L.host.data(), bytes, hipMemcpyHostToDevice),
            "expert table copy");
+    L.resident = 0;
+    for (const Dsv4ExpertDev &e : L.host) L.resident += e.w1 != nullptr;
     L.dirty = false;
     return 0;
 }
@@ -1089,7 +1092,8 @@ int dsv4_gpu_moe_fp4_n(float *out, const float *x, int layer, const int *idx,
                                     inter, swiglu_limit, g_moe.p, g_stream) != 0)
                 return -1;
     } else if (dsv4_moe_fp4_n_launch((float *)out_at(oo), (const float *)(g_ar.d + xo),
-                                     L->dev, (int)L->host.size(), (const int *)(g_ar.d + io),
+                                     L->dev, (int)L->host.size(), L->resident,
+                                     (const int *)(g_ar.d + io),
                                      (const float *)(g_ar.d + wo), nt, topk, hidden, inter,
                                      swiglu_limit, g_moe.p, g_stream) != 0) {
         return -1;
@@ -1109,8 +1113,8 @@ int dsv4_gpu_moe_fp4_n_d(float *d_out, const float *d_x, int layer, const int *d
     if (moe_prepare(layer, topk, hidden, inter, &L) != 0) return -1;
     if (scratch_reserve(g_moe, dsv4_moe_n_scratch_bytes(nt, topk, hidden, inter)) != 0)
         return -1;
-    return dsv4_moe_fp4_n_launch(d_out, d_x, L->dev, (int)L->host.size(), d_idx, d_w, nt,
-                                 topk, hidden, inter, swiglu_limit, g_moe.p,
+    return dsv4_moe_fp4_n_launch(d_out, d_x, L->dev, (int)L->host.size(), L->resident, d_idx,
+                                 d_w, nt, topk, hidden, inter, swiglu_limit, g_moe.p,
                                  as_stream(stream));
 }
 

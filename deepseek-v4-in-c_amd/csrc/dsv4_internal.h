@@ -211,14 +211,16 @@ int dsv4_moe_fp4_launch(float *d_out, const float *d_x,
                         hipStream_t st);
 
 /* Batched routed MoE (prefill, the routed half of moe_n): d_out[nt][hidden]
- * for d_x[nt][hidden], routing d_idx/d_w [nt][topk]; each distinct expert's
- * weights stream once for the batch and every token's row is bit-identical
- * to dsv4_moe_fp4_launch on that token. Scratch of dsv4_moe_n_scratch_bytes
- * (at least dsv4_moe_scratch_bytes). */
+ * for d_x[nt][hidden], routing d_idx/d_w [nt][topk], d_table's n_table entries
+ * holding n_experts experts; each distinct expert's weights stream once for
+ * the batch and every token's row is bit-identical to dsv4_moe_fp4_launch on
+ * that token. Scratch of dsv4_moe_n_scratch_bytes (at least
+ * dsv4_moe_scratch_bytes). */
 size_t dsv4_moe_n_scratch_bytes(int nt, int topk, int hidden, int inter);
 int dsv4_moe_fp4_n_launch(float *d_out, const float *d_x, const Dsv4ExpertDev *d_table,
-                          int n_table, const int *d_idx, const float *d_w, int nt, int topk,
-                          int hidden, int inter, float limit, void *scratch, hipStream_t st);
+                          int n_table, int n_experts, const int *d_idx, const float *d_w,
+                          int nt, int topk, int hidden, int inter, float limit, void *scratch,
+                          hipStream_t st);
 
 /* The VALU form; hbuf is device scratch [topk][inter] f32. */
 int dsv4_moe_fp4_valu_launch(float *d_out, const float *d_x,

@@ -1554,8 +1554,9 @@ size_t dsv4_moe_n_scratch_bytes(int nt, int topk, int hidden, int inter)
 }
 
 int dsv4_moe_fp4_n_launch(float *d_out, const float *d_x, const Dsv4ExpertDev *d_table,
-                          int n_table, const int *d_idx, const float *d_w, int nt, int topk,
-                          int hidden, int inter, float limit, void *scratch, hipStream_t st)
+                          int n_table, int n_experts, const int *d_idx, const float *d_w,
+                          int nt, int topk, int hidden, int inter, float limit, void *scratch,
+                          hipStream_t st)
 {
     if (nt < 1 || topk < 1) return -1;
     const int form = mc_env("DSV4_GPU_MOE_MC", 2);
@@ -1585,13 +1586,13 @@ int dsv4_moe_fp4_n_launch(float *d_out, const float *d_x, const Dsv4ExpertDev *d
     const dim3 ga(inter / 32, slots), gb(hidden / 64, slots);
     const uint32_t xb = (uint32_t)((size_t)nt * MC_NT * hidden * 2);
     const uint32_t hb = (uint32_t)((size_t)np * MC_NT * inter * 2);
-    /* a second column tile per pass where the experts average more than its
-     * five pairs, so that most take one pass over their weights; its LDS (81
-     * against 50 KB) leaves two workgroups per CU instead of three (us, two /
-     * one tile, 7168 x 2048, top 8: 64 tokens of 64 experts 524 / 627, of 16
-     * 461 / 594; 32 tokens of 64 experts 390 / 368, 64 tokens of 256 1165 /
-     * 967; three tiles 571, 470, 443, 1356) */
-    const int ctm = np > 5 * n_table ? 2 : 1;
+    /* a second column tile per pass where the layer's experts, whatever their
+     * ids, average more than its five pairs, so that most take one pass over
+     * their weights; its LDS (81 against 50 KB) leaves two workgroups per CU
+     * instead of three (us, two / one tile, 7168 x 2048, top 8: 64 tokens of
+     * 64 experts 524 / 627, of 16 461 / 594; 32 tokens of 64 experts 390 /
+     * 368, 64 tokens of 256 1165 / 967; three tiles 571, 470, 443, 1356) */
+    const int ctm = np > 5 * n_experts ? 2 : 1;
     static bool opted = false;
     if (!opted) {
         mc_lds_optin(k_mn_pass<2, 14, true, 1>); mc_lds_optin(k_mn_pass<3, 0, true, 1>);

@@ -128,3 +128,22 @@ def test_route_moe(tmp_path, mode):
     shapes = [s if mode is None else s[:-1] + (mode == "0",) for s in MOE_SHAPES]
     env = {} if mode is None else {"DSV4_GPU_MOEN_TOKENWISE": mode}
     assert hip_shim.run(tmp_path, MOE.replace("SHAPES", repr(shapes)), env).endswith("ok\n")
+
+
+TILES = MOE.split("for layer")[0].replace("range(64)", "range(first, first + n)").replace(
+    "def batched(layer,", "def two_tiles(first, n, layer,").replace("layer, 0)", "layer, first)").replace(
+    "% distinct", "% distinct + first").replace("k_mn_prepare", "ELi2EEEvPvPKt") + r"""
+for layer, (first, n, nt, want) in enumerate(SHAPES):
+    assert two_tiles(first, n, layer, 4096, 1024, 8, nt, n) == want, (first, n, nt)
+print("ok")
+"""
+
+# experts first .. first + n - 1 of a layer, nt tokens of top 8: two column tiles a
+# pass where the resident experts average more than five pairs, wherever their ids lie
+TILE_SHAPES = [(0, 32, 64, True), (1000, 32, 64, True), (1000, 32, 20, False), (0, 32, 20, False),
+               (0, 128, 64, False), (200, 8, 6, True)]
+
+
+def test_two_tiles_by_experts(tmp_path):
+    child = TILES.replace("SHAPES", repr(TILE_SHAPES))
+    assert hip_shim.run(tmp_path, child).endswith("ok\n")

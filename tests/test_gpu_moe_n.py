@@ -11,7 +11,8 @@ Bars:
     compiled reference's batched FP4 matmul).
 Routing draws every token's experts from a small pool, so experts repeat
 across the batch (the union the reference builds) and some get more pairs
-than one 5-pair pass of the kernel takes.
+than one pass of the kernel takes (5 pairs, or 10 where the layer's experts
+average more than 5).
 """
 import ctypes
 
@@ -90,9 +91,7 @@ def test_moe_n_c3_shape(gpu, dsv4, nt):
 
 def test_moe_n_one_expert_set_for_every_token(gpu, dsv4):
     """64 tokens that all ask for the same 8 experts: 64 pairs per expert, so
-    each expert runs 7 passes of up to 10 pairs over its weights. (The ids lie
-    below 32, so 512 pairs are more than five per table entry: two column
-    tiles a pass.)"""
+    each expert runs 7 passes of up to 10 pairs over its weights."""
     rng, table = _setup(dsv4, 6, 7168, 2048, 8, 7)
     IDX, W, X = _batch(rng, table, 64, 8, 7168, same=True)
     _check(dsv4, 6, table, IDX, W, X, 7168, 2048, 10.0, oracle_tokens=[0, 33, 63])

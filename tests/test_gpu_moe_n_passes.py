@@ -37,11 +37,10 @@ def _check(dsv4, layer, X, IDX, W, hidden, inter):
 @pytest.mark.parametrize("layer,hidden,inter", [(310, 7168, 2048), (311, 512, 512),
                                                 (312, 2560, 1024)])
 def test_pairs_per_expert(gpu, dsv4, monkeypatch, layer, hidden, inter):
-    """Expert e of 12 is asked for by e + 1 tokens (78 pairs: one tile per
-    pass; the other experts make the table large enough)."""
+    """Expert e of 12 is asked for by e + 1 tokens (78 pairs, and 16 experts in
+    the layer: at most five each on average, so one tile per pass)."""
     monkeypatch.setenv("DSV4_GPU_MOEN_TOKENWISE", "0")
-    # ids 0..11 used, 31 sets the table's size
-    rng = _experts(gpu, dsv4, layer, list(range(12)) + [31], hidden, inter, 5)
+    rng = _experts(gpu, dsv4, layer, list(range(15)) + [31], hidden, inter, 5)
     pairs = [e for e in range(12) for _ in range(e + 1)]
     IDX = np.array(pairs, np.int32).reshape(39, 2)
     IDX[:, 1] = np.roll(IDX[:, 1], 7)
