@@ -1142,13 +1142,13 @@ def main():
                 "frac_bf16_peak": round(gf64 / us * 1e3 / 2500.0, 4),
                 "us_per_token": round(us / 64, 3),
                 "scales": "E8M0, " + ("matrix-core form (DSV4_GPU_FP8_MX=1)" if form == "1"
-                                      else "VALU form (the default)"),
+                                      else "the default form (k_batch_mf from 5 tokens)"),
                 "by_tokens": curve}
         os.environ.pop("DSV4_GPU_FP8_MX", None)
         us32, _ = B.gemv_n_run(nt=64, sfmt=1)
         detail["prefill_fp8_7168x7168_nt64_f32_scales"] = {
             "us": round(us32, 3), "TFLOPs": round(gf64 / us32 * 1e3, 2),
-            "frac_fp32_peak": round(gf64 / us32 * 1e3 / 157.3, 4), "scales": "fp32 (VALU form)"}
+            "frac_fp32_peak": round(gf64 / us32 * 1e3 / 157.3, 4), "scales": "fp32 (k_batch_mf)"}
         log("bench: host-buffer call cost fit (dsv4_gpu_mmq, 10 shapes)")
         detail["host_call_fit"] = B.host_call_fit()
         for ratio, name in ((4, "attn_block_flash_csa_ratio4"), (128, "attn_block_flash_hca_ratio128")):

@@ -1200,10 +1200,11 @@ __device__ __forceinline__ v4f term_sum_at(const v4f &d, int lane, int c0)
  * the next copies and weights requested, the unit's products.
  *
  * What bounds it: the weight stream. C3's expert shape, 64 tokens of 256
- * experts, us per call: 1155 with all 16 term rows of a tile brought through
- * registers per unit whatever the pass's pairs, 967 with this; 914 with the
- * terms left out altogether and 864 (6.1 TB/s) with the products left out
- * too. D = 3 or 4 weight units in flight measured the same (966, 993). */
+ * experts, us per call: 1131 with all 16 term rows of a tile brought through
+ * registers per unit whatever the pass's pairs, 933 with this. In another run,
+ * where this took 967: 914 with the terms left out altogether, 864 (6.1 TB/s)
+ * with the products left out too, 966 and 993 with D = 3 and 4 weight units
+ * in flight. */
 template <int D, int NU, int CT, int RPW>
 __device__ __forceinline__ void mn_units(v4f *res, const uint16_t *src, uint32_t src_bytes,
                                          const int *prow, int nb, int K, const uint8_t *base,
@@ -1591,7 +1592,8 @@ int dsv4_moe_fp4_n_launch(float *d_out, const float *d_x, const Dsv4ExpertDev *d
      * their weights; its LDS (81 against 50 KB) leaves two workgroups per CU
      * instead of three (us, two / one tile, 7168 x 2048, top 8: 64 tokens of
      * 64 experts 524 / 627, of 16 461 / 594; 32 tokens of 64 experts 390 /
-     * 368, 64 tokens of 256 1165 / 967; three tiles 571, 470, 443, 1356) */
+     * 368, 64 tokens of 256 1165 / 967; three tiles 571, 470, 443, 1356; all
+     * in one run, see mn_units) */
     const int ctm = np > 5 * n_experts ? 2 : 1;
     static bool opted = false;
     if (!opted) {

@@ -248,14 +248,14 @@ def _same_bits_or_nan(a, b):
 @pytest.mark.parametrize("scales", ["e8m0", "f32"])
 @pytest.mark.parametrize("slots", ["0", "16", "32", "64"])
 def test_batched_matrix_core_f32_chains_keep_bits(gpu, dsv4, monkeypatch, slots, scales):
-    """The batched kernel for columns a multiple of 64 (k_fp8_mfn) runs the
-    GEMV's four fmaf chains per chunk on v_mfma_f32_16x16x4f32 and the rest
-    of its arithmetic on the VALU. Against the single-token GEMV and the VALU
-    batched kernel (DSV4_GPU_FP8_MFN=0), bit for bit, for every part size
-    DSV4_GPU_MFN_L (0: the launcher's rule, which keeps small batches and
-    small launches on the VALU kernel; a size a shape does not take falls
-    back to the VALU kernel), both scale formats, 16 to 256 row slots (1024
-    to 16384 columns, and 512 = 32 slots), 1 to 4 chunks per slot, ragged
+    """The matrix-core batched kernel (k_batch_mf) runs the GEMV's four fmaf
+    chains per chunk on v_mfma_f32_16x16x4f32 and the rest of its arithmetic
+    on the VALU. Against the single-token GEMV and the VALU batched kernel
+    (DSV4_GPU_FP8_MFN=0), bit for bit, for every number of slots per wave
+    DSV4_GPU_MFN_L (0: the launcher's rule, which keeps small batches on the
+    VALU kernel and splits tiles over workgroups; a number a shape does not
+    take falls back to the VALU kernel), both scale formats, 16 to 256 row
+    slots (256 to 16384 columns), 1 to 4 chunks per slot, ragged
     row tiles and token tiles, a token of signed zeros against zero codes of
     both signs, a token of subnormals, and a token with inf."""
     cases = ((300, 1536, 5), (129, 7168, 37), (70, 16384, 2), (33, 4096, 17), (18, 3072, 7),

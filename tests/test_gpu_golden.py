@@ -47,9 +47,11 @@ GM = np.load(os.path.join(HERE, "golden", "golden_fp8n_mc.npz"))
 def test_fp8_batched_matrix_core_golden(gpu, dsv4, monkeypatch, slots):
     """The compiled reference's dsv4_matmul_fp8_n at 192x1024, 17 tokens,
     against mmq_n on the f32 matrix-core batched kernel (DSV4_GPU_MFN_L
-    16 / 32 / 64: four, two or one part per row, with and without the join)
-    and on the launcher's rule (0: this small launch takes the VALU kernel):
-    within 1e-5, and every token bit-identical to the single-token GEMV."""
+    16 / 32 / 64: four, two or one wave per row tile; 0, the launcher's rule:
+    sixteen). Forced numbers are never split over workgroups and the rule
+    splits rows of 4096 columns on, so none of these joins (the split tiles:
+    test_gpu_batch_mf.py). Within 1e-5, and every token bit-identical to the
+    single-token GEMV."""
     W, S, x = GM["W"], GM["S"], GM["x"]
     _keep.extend([W, S])
     m = dsv4.qmat(W, S)
