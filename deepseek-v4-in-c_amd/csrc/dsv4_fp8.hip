@@ -189,17 +189,28 @@ __device__ __forceinline__ void load_step(u32x4 (*wv)[NCH], uint32_t *sv, const 
  * x does not wait for the first weights; but each form was measured, cold, us:
  *   - E8M0, x from L2: decoded and held (7168x12288 17.67 -> 17.09, 7168x7168
  *     12.12 -> 11.69), but raw for three chunks and one row per step without
- *     prefetch (4096x9216 12.71 -> 11.08, 5120x4608 8.91 -> 7.92);
+ *     prefetch (4096x9216 12.71 -> 11.08, 5120x4608 8.91 -> 7.92) or two rows
+ *     with it (3426x8464 10.67 -> 9.91), and raw and free for four chunks and
+ *     two rows with prefetch (rows of 192 and 256 threads: 0.98 to 1.00 and
+ *     0.97 to 0.99 times);
  *   - fp32, x from L2: held for one row per step (7168x7168 11.84 -> 11.50),
- *     not for more (16384x12288 35.7 -> 34.2, 1536x12288 8.11 -> 7.90);
+ *     for four, and for three chunks with prefetch (0.98 and 0.99 times), not
+ *     for two rows else (16384x12288 35.7 -> 34.2, 1536x12288 8.11 -> 7.90);
+ *   - rows of 128 threads through LDS, E8M0, four chunks, two rows per step
+ *     without prefetch: decoded and held (10164x7824 16.86 -> 15.78);
  *   - rows of 256 threads through LDS: E8M0 decoded without prefetch
  *     (7168x16384 21.65 -> 20.95), raw with it (4096x16384 14.21 -> 14.05);
  *     fp32 held with prefetch (7168x16384 21.42 -> 20.77, 4096x16384 14.6 ->
  *     14.1), free in one step (256x16384 4.74 -> 4.19). */
 template <int NCH, int R, int SF, int PF, int XL>
 struct Fp8Form {
-    static constexpr bool RAW = XL == 0 ? NCH == 3 && R == 1 && !PF : XL != 4 || PF;
-    static constexpr bool HELD = XL == 0 ? SF == 0 || R == 1 : XL == 4 && SF == 1 && PF;
+    static constexpr bool TWO_PF = R == 2 && PF;
+    static constexpr bool X2 = XL == 2 && SF == 0 && NCH == 4 && R == 2 && !PF;
+    static constexpr bool RAW = XL == 0 ? (NCH == 3 && R == 1 && !PF) || (NCH >= 3 && TWO_PF)
+                                        : (XL != 4 || PF) && !X2;
+    static constexpr bool HELD = XL != 0 ? X2 || (XL == 4 && SF == 1 && PF)
+                               : SF == 0 ? !(NCH == 4 && TWO_PF)
+                                         : R != 2 || (NCH == 3 && PF);
 };
 
 /* One workgroup owns the contiguous rows [row0, row0 + rows_per_wg). It walks
@@ -569,7 +580,7 @@ struct Fp8Plan {
 };
 
 /* Whether a row's x goes through LDS, one fetch per workgroup instead of one
- * per row group (steps: a workgroup's). Rows of up to 64 threads: always (us,
+ * per row group (steps: a workgroup's; wgs: the launch's workgroups). Rows of up to 64 threads: always (us,
  * cold, each thread its own x from L2 / through LDS: 4096x4096 5.99 / 5.57,
  * 512x4096 3.73 / 3.28, 32768x4096 25.0 / 23.6, 24576x1536 9.68 / 9.25). Wider
  * rows have fewer row groups to share it, and each group's rounds of 1024
@@ -577,15 +588,19 @@ struct Fp8Plan {
  *   - 128 threads, E8M0: where a step has four rows or the next one is
  *     prefetched (1536x7168 5.71 / 5.56, 2560x4608 6.51 / 5.93), or four
  *     chunks fill the rounds (2048x8192 6.63 / 6.30; 7168x7168 11.7 / 12.0,
- *     8192x4608 9.44 / 9.85, 1024x4608 3.96 / 4.39);
+ *     8192x4608 9.44 / 9.85, 1024x4608 3.96 / 4.39) or, two rows per step, up to
+ *     three workgroups for two CUs (4435x7104 10.05 / 9.67, 5786x6240 9.60 / 10.10);
  *   - 128 threads, fp32: not for one row per step (512x4608 3.58 / 3.79,
  *     5120x4608 7.70 / 8.18), but where four chunks fill the rounds (512x8192
- *     3.95 / 3.77), and with prefetch where the rounds are full or there are
- *     four chunks (4096x5120 6.92 / 7.19; 2048x7168 6.03 / 5.93);
- *   - 256 threads: but for single steps whose rounds are not full (256x13312
- *     fp32 4.05 / 4.39; 4096x13312 14.5 / 12.2, 1024x16384 7.4 / 6.8).
+ *     3.95 / 3.77), with prefetch where the rounds are full or there are
+ *     four chunks (4096x5120 6.92 / 7.19; 2048x7168 6.03 / 5.93), and for three
+ *     chunks without prefetch from four steps on (5823x5200 8.40 / 8.60);
+ *   - 256 threads: where a workgroup has several steps or a CU several
+ *     workgroups, which then want x at once (4096x13312 14.5 / 12.2, E8M0
+ *     936x14400 7.02 / 6.63, 1024x16384 7.4 / 6.8; 199x15664 4.69 / 4.86, fp32
+ *     78x15680 4.01 / 4.20, and 3.72 / 4.25 with W in the Infinity Cache).
  * Rows of 192 threads, whose workgroup is not 256, read it from L2. */
-bool fp8_xl(const Fp8Geom &g, int R, int pf, int sfmt, int cols, int steps)
+bool fp8_xl(const Fp8Geom &g, int R, int pf, int sfmt, int cols, int steps, int wgs)
 {
     if (g.wg != 256 || (cols & 3)) return false;
     const int waves = g.tc > 64 ? g.tc / 64 : 1;
@@ -593,9 +608,10 @@ bool fp8_xl(const Fp8Geom &g, int R, int pf, int sfmt, int cols, int steps)
     bool xl = true;
     if (waves == 2)
         xl = R == 4 || (g.nch == 4 && full) ||
-             (sfmt == 0 ? pf != 0 : R == 2 && (!pf || full || g.nch == 4));
+             (sfmt == 0 ? pf != 0 || (g.nch == 4 && R == 2 && wgs * 2 <= 3 * cu_count())
+                        : R == 2 && (g.nch == 4 || (pf ? full : steps >= 4)));
     else if (waves == 4)
-        xl = full || steps > 1;
+        xl = steps > 1 || wgs > cu_count();
     return env_int("DSV4_GPU_FP8_XL", xl) != 0;
 }
 
@@ -613,7 +629,7 @@ Fp8Plan fp8_plan(const Fp8Geom &g, int R, int pf, int sfmt, int rows, int cols, 
     if (spw < 1) spw = 1;
     p.rows_per_wg = spw * step_rows;
     p.grid = (rows + p.rows_per_wg - 1) / p.rows_per_wg;
-    p.xl = lds_x && fp8_xl(g, R, pf, sfmt, cols, spw);
+    p.xl = lds_x && fp8_xl(g, R, pf, sfmt, cols, spw, p.grid * ngroups);
     p.lds = (g.tc > 64 ? sizeof(float) * (size_t)wpr * p.rows_per_wg : 0)
           + (p.xl ? sizeof(float) * (size_t)cols : 0);
     return p;

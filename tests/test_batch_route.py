@@ -1,7 +1,8 @@
 """Which kernels a batched call takes, at shapes where both were timed, on both
 sides of the rules' lines: FP4 and BF16 (us, matrix core / VALU kernel), FP8 with
 and without a place for part sums, and the routed experts' host call (batched /
-token by token). CPU only."""
+token by token); and whether a single-token FP8 GEMV's x goes through LDS. CPU
+only."""
 import pytest
 
 import hip_shim
@@ -71,7 +72,8 @@ print("ok")
 
 # on a stream with a place for part sums, and captured, where tiles stay whole
 # (us, whole tiles / VALU): 14.8 / 13.2, 14.8 / 14.2, 1.16 and 0.77 times, 21.2 /
-# 13.4 at 10240 columns, 24.7 / 22.7, 25.2 / 27.9, 27.2 / 24.9, 27.6 / 28.9, 30.8 / 29.9, 11.2 / 15.2
+# 13.4 at 10240 columns, 24.7 / 22.7, 25.2 / 27.9, 27.2 / 24.9, 27.6 / 28.9, 30.8 /
+# 29.9, 11.2 / 15.2
 FP8_SHAPES = [
     (512, 6144, 5, True, False), (512, 6144, 7, True, True), (512, 4112, 8, True, False),
     (512, 4112, 9, True, True), (64, 11264, 12, True, False), (512, 12288, 12, True, False),
@@ -131,8 +133,9 @@ def test_route_moe(tmp_path, mode):
 
 
 TILES = MOE.split("for layer")[0].replace("range(64)", "range(first, first + n)").replace(
-    "def batched(layer,", "def two_tiles(first, n, layer,").replace("layer, 0)", "layer, first)").replace(
-    "% distinct", "% distinct + first").replace("k_mn_prepare", "ELi2EEEvPvPKt") + r"""
+    "def batched(layer,", "def two_tiles(first, n, layer,").replace(
+    "layer, 0)", "layer, first)").replace("% distinct", "% distinct + first").replace(
+    "k_mn_prepare", "ELi2EEEvPvPKt") + r"""
 for layer, (first, n, nt, want) in enumerate(SHAPES):
     assert two_tiles(first, n, layer, 4096, 1024, 8, nt, n) == want, (first, n, nt)
 print("ok")
@@ -146,4 +149,28 @@ TILE_SHAPES = [(0, 32, 64, True), (1000, 32, 64, True), (1000, 32, 20, False), (
 
 def test_two_tiles_by_experts(tmp_path):
     child = TILES.replace("SHAPES", repr(TILE_SHAPES))
+    assert hip_shim.run(tmp_path, child).endswith("ok\n")
+
+
+GEMV = CHILD.split("def route")[0] + r"""
+for rows, cols, sf, xl in SHAPES:
+    shim.shim_reset(-1, 0)
+    assert L.dsv4_gpu_fp8_gemv_d(a, a, a, a, sf, rows, cols, None) == 0
+    n = shim.shim_kernel(0)
+    assert n.split(b"k_fp8_gemvILi")[1].split(b"E")[4] == b"Li%d" % xl, (rows, cols, sf, n)
+print("ok")
+"""
+
+# rows, cols, scales, the waves of a row whose x goes through LDS or 0 (us, cold, own
+# loads / through LDS): 4.01 / 4.20, 4.69 / 4.86, 7.02 / 6.63, 14.5 / 12.2, 7.4 / 6.8,
+# 8.40 / 8.60, 5.99 / 5.57, 11.7 / 12.0, 6.63 / 6.30, 10.05 / 9.67, 9.60 / 10.10
+GEMV_SHAPES = [
+    (78, 15680, 1, 0), (199, 15664, 0, 0), (936, 14400, 0, 4), (4096, 13312, 1, 4),
+    (1024, 16384, 0, 4), (5823, 5200, 1, 0), (20000, 5200, 1, 2), (4096, 4096, 0, 1),
+    (7168, 7168, 0, 0), (2048, 8192, 0, 2), (4435, 7104, 0, 2), (5786, 6240, 0, 0),
+]
+
+
+def test_x_through_lds(tmp_path):
+    child = GEMV.replace("SHAPES", repr(GEMV_SHAPES))
     assert hip_shim.run(tmp_path, child).endswith("ok\n")
