@@ -190,7 +190,7 @@ __device__ __forceinline__ void load_step(u32x4 (*wv)[NCH], uint32_t *sv, const 
  *   - E8M0, x from L2: decoded and held (7168x12288 17.67 -> 17.09, 7168x7168
  *     12.12 -> 11.69), but raw for three chunks and one row per step without
  *     prefetch (4096x9216 12.71 -> 11.08, 5120x4608 8.91 -> 7.92) or two rows
- *     with it (3426x8464 10.67 -> 9.91), and raw and free for four chunks and
+ *     with it (3426x8464 10.67 -> 9.67), and raw and free for four chunks and
  *     two rows with prefetch (rows of 192 and 256 threads: 0.98 to 1.00 and
  *     0.97 to 0.99 times);
  *   - fp32, x from L2: held for one row per step (7168x7168 11.84 -> 11.50),
@@ -597,7 +597,7 @@ struct Fp8Plan {
  *     chunks without prefetch from four steps on (5823x5200 8.40 / 8.60);
  *   - 256 threads: where a workgroup has several steps or a CU several
  *     workgroups, which then want x at once (4096x13312 14.5 / 12.2, E8M0
- *     936x14400 7.02 / 6.63, 1024x16384 7.4 / 6.8; 199x15664 4.69 / 4.86, fp32
+ *     936x14400 7.02 / 6.64, 1024x16384 7.4 / 6.8; 199x15664 4.69 / 4.86, fp32
  *     78x15680 4.01 / 4.20, and 3.72 / 4.25 with W in the Infinity Cache).
  * Rows of 192 threads, whose workgroup is not 256, read it from L2. */
 bool fp8_xl(const Fp8Geom &g, int R, int pf, int sfmt, int cols, int steps, int wgs)

@@ -162,7 +162,7 @@ print("ok")
 """
 
 # rows, cols, scales, the waves of a row whose x goes through LDS or 0 (us, cold, own
-# loads / through LDS): 4.01 / 4.20, 4.69 / 4.86, 7.02 / 6.63, 14.5 / 12.2, 7.4 / 6.8,
+# loads / through LDS): 4.01 / 4.20, 4.69 / 4.86, 7.02 / 6.64, 14.5 / 12.2, 7.4 / 6.8,
 # 8.40 / 8.60, 5.99 / 5.57, 11.7 / 12.0, 6.63 / 6.30, 10.05 / 9.67, 9.60 / 10.10
 GEMV_SHAPES = [
     (78, 15680, 1, 0), (199, 15664, 0, 0), (936, 14400, 0, 4), (4096, 13312, 1, 4),
